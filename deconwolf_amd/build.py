@@ -23,6 +23,9 @@ LIB = os.path.join(HERE, "libdwhip.so")
 
 N_XMODES = 7
 N_CMODES = 9
+# modes compiled for extended jobs too (xmode_has_ext, cmode_has_ext)
+EXT_XMODES = (1, 2, 3, 4)
+EXT_CMODES = (0, 1, 3, 4, 7, 8)
 
 # -packed-fp32-ops: no packed FP32 instructions in device code.  The host
 # pass of hipcc warns that it does not know the feature; that is harmless.
@@ -45,8 +48,12 @@ def units():
     u = []
     for m in range(N_XMODES):
         u.append(("k_xpass.hip", ["-DXMODE=%d" % m], "k_xpass_%d.o" % m))
+    for m in EXT_XMODES:
+        u.append(("k_xpass.hip", ["-DXMODE=%d" % m, "-DPASS_EXT"], "k_xpass_e%d.o" % m))
     for m in range(N_CMODES):
         u.append(("k_colpass.hip", ["-DCMODE=%d" % m], "k_colpass_%d.o" % m))
+    for m in EXT_CMODES:
+        u.append(("k_colpass.hip", ["-DCMODE=%d" % m, "-DPASS_EXT"], "k_colpass_e%d.o" % m))
     u.append(("k_misc.hip", [], "k_misc.o"))
     u.append(("k_output.hip", [], "k_output.o"))
     u.append(("k_bw.hip", [], "k_bw.o"))

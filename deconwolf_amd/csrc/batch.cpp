@@ -166,10 +166,10 @@ void table_free(Table* t)
 // Fills t with jobs and queues its upload on s.
 // REL/ABS jobs of the fused passes stop on the device: the end-of-round
 // kernel applies dw_iterator_next and the passes skip a stopped job, so
-// such jobs join multi-round steps; any-size jobs decide on the host
+// such jobs join multi-round steps; extended and any-size jobs decide on the host
 bool dev_stop_job(const EngJob* j)
 {
-    return j->prm.iter_type != DWHIP_ITER_FIXED && !j->j.generic;
+    return j->prm.iter_type != DWHIP_ITER_FIXED && !dwhip_job_solo(&j->j);
 }
 
 int table_build(Table* t, const std::vector<EngJob*>& jobs, hipStream_t s)
@@ -206,8 +206,8 @@ int table_pass(const Table& t, bool xkind, int mode, hipStream_t s)
     const int kind = xkind ? xmode_kind(mode) : cmode_kind(mode);
     if (t.n == 0 || t.ntile[kind] == 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    hipError_t e = xkind ? dwhip_launch_xpass(mode, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s)
-                         : dwhip_launch_colpass(mode, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
+    hipError_t e = xkind ? dwhip_launch_xpass(mode, 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s)
+                         : dwhip_launch_colpass(mode, 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
     if (slot >= 0) {
         double by = 0;
         for (EngJob* j : t.jobs) by += dwhip_pass_bytes(xkind ? 1 : 0, mode, j->j.d, j->j.host_iter);
@@ -300,10 +300,10 @@ int setup(dwhip_engine* E, const std::vector<EngJob*>& fresh)
 {
     if (fresh.empty()) return DWHIP_OK;
     hipStream_t s = E->s;
-    // jobs on the any-size path set up one by one; the others batched
+    // extended and any-size jobs set up one by one; the others batched
     std::vector<EngJob*> fast;
     for (EngJob* j : fresh) {
-        if (j->j.generic)
+        if (dwhip_job_solo(&j->j))
             RCHK(dwhip_job_setup(&j->j, s));
         else
             fast.push_back(j);
@@ -461,6 +461,11 @@ int dwhip_engine_submit(dwhip_engine* E, const float* im, int64_t M, int64_t N, 
     j->out = out;
     const float* start = prm->start != DWHIP_START_FLAT ? prm->start_image : nullptr;
     int rc = dwhip_job_plan(&j->j, im, M, N, P, psf, pM, pN, pP, prm, start);
+    if (rc == DWHIP_OK && align_up(j->j.bytes, 4096) > E->cfg.hbm_budget && j->j.ext) {
+        // the any-size path needs less (no padded spectra)
+        j->j.allow_ext = false;
+        rc = dwhip_job_plan(&j->j, im, M, N, P, psf, pM, pN, pP, prm, start);
+    }
     if (rc == DWHIP_OK && align_up(j->j.bytes, 4096) > E->cfg.hbm_budget) rc = DWHIP_ERR_NOMEM;
     if (rc != DWHIP_OK) {
         delete j;
@@ -520,9 +525,11 @@ static int group_round(Table* tae, Table* tfh, const std::vector<EngJob*>& all, 
     for (EngJob* j : all) {
         const bool fixed = j->prm.iter_type == DWHIP_ITER_FIXED;
         const bool full = !fixed || j->j.d.rl || j->j.host_iter + 1 < j->prm.niter;
-        if (j->j.generic) {
-            // the any-size path runs its own passes, one job at a time
-            RCHK(dwhip_generic_round(&j->j, full, s));
+        if (dwhip_job_solo(&j->j)) {
+            // extended and any-size jobs run their own passes, one at a time
+            // (the step counts the round for every job)
+            RCHK(dwhip_job_round(&j->j, full, s));
+            j->j.host_iter -= 1;
             continue;
         }
         jobs.push_back(j);
@@ -581,15 +588,15 @@ static int capture_round(void* ctx, hipStream_t cs)
 // Rounds this step runs: up to the next known completion (the fewest
 // rounds any job has left before nIter, or maxiter for REL/ABS jobs, which
 // may stop earlier on the device), at most rounds_per_step; one round with
-// an any-size job active (its REL/ABS rule runs on the host after each
-// round) and while kernels are profiled (events per pass).
+// an extended or any-size job active (its REL/ABS rule runs on the host after
+// each round) and while kernels are profiled (events per pass).
 static int step_rounds(const dwhip_engine* E)
 {
     const int cap = std::max(1, E->cfg.rounds_per_step);
     if (cap == 1 || dwhip_prof_on() || dwhip_graph_mode() == 0) return 1;
     int r = cap;
     for (const EngJob* j : E->active) {
-        if (j->j.generic) return 1;
+        if (dwhip_job_solo(&j->j)) return 1;
         r = std::min(r, iter_target(j) - j->j.host_iter);
     }
     return std::max(1, r);

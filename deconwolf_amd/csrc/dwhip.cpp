@@ -142,6 +142,42 @@ bool dwhip_fast_size_ok(const int64_t* w)
     return true;
 }
 
+// Transform lengths L of an extended job: a work size w the fused passes
+// cannot transform, its circular convolution of period w[d] computed as one
+// of length L[d] >= w[d] + p[d] - 1 that they can (an axis they transform at
+// w[d] keeps it).  Against the any-size path (Bluestein, a pair of length
+// >= 2 w[d] - 1 transforms per axis, elementwise steps unfused), ten iterations
+// of 1115 x 1115 x 100 with a 181 x 181 x 79 PSF, transformed at 1296 x 1296 x
+// 100, take 36.5 ms instead of 153.7.  False when an axis has no such length or its PSF is
+// longer than the period (the any-size path then runs the job).
+bool dwhip_ext_size(const int64_t* w, int64_t pM, int64_t pN, int64_t pP, int64_t* L)
+{
+    const int64_t p[3] = {pM, pN, pP};
+    for (int d = 0; d < 3; ++d) {
+        if (w[d] < 1 || w[d] > (1 << 20) || p[d] > w[d]) return false;
+        int64_t t[3] = {2, 1, 1};
+        t[d] = w[d];
+        if (dwhip_fast_size_ok(t)) {
+            L[d] = w[d];
+            continue;
+        }
+        const int64_t need = w[d] + p[d] - 1;
+        // the searches below end: every axis plans some length up to its limit
+        const int64_t limit = d == 0 ? 2 * DWHIP_XMAXE * DWHIP_XTHR : d == 1 ? DWHIP_YMAXE * DWHIP_CTHR
+                                                                             : DWHIP_ZMAXE * DWHIP_ZTHR;
+        L[d] = 0;
+        for (int64_t n = need; n <= limit; ++n) {
+            t[d] = n;
+            if (dwhip_fast_size_ok(t)) {
+                L[d] = n;
+                break;
+            }
+        }
+        if (L[d] == 0) return false;
+    }
+    return dwhip_fast_size_ok(L);
+}
+
 int dwhip_work_size(int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN, int64_t pP,
                     int border_quality, int64_t* work, int64_t* ref_work)
 {
@@ -334,6 +370,21 @@ static size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN,
                        int64_t pP, int border_quality, int niter)
 {
+    int64_t L[3];
+    if (!dwhip_fast_size_ok(work) && dwhip_ext_size(work, pM, pN, pP, L)) {
+        // extended job: spectra of the transform's rows and columns (C in the
+        // data's planes, K in all), U0, U1 (and W) of the data
+        const size_t hcs = round_up(L[0] / 2 + 1, 16);
+        const size_t V = round_up(work[0], 2) * work[1] * work[2];
+        DwhipTiles t;
+        dwhip_tile_config(L, &t);
+        size_t b = hcs * L[1] * (work[2] + L[2]) * sizeof(float2) + (border_quality > 0 ? 3 : 2) * V * sizeof(float);
+        b += (size_t)ratio_tiles(work[1], work[2], t.xrows) * sizeof(double);
+        b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
+        b += DWHIP_STAT_BLOCKS * 4 * sizeof(double) + 4096 + 2 * sizeof(JobDev);
+        for (int d = 0; d < 3; ++d) b += 3 * (size_t)L[d] * sizeof(float2);
+        return b;
+    }
     if (!dwhip_fast_size_ok(work)) {
         // any-size path: half spectra Z and K, U0, U1 (and W), partials, tables
         const size_t V = (size_t)work[0] * work[1] * work[2];
@@ -355,7 +406,7 @@ size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int
     b += (size_t)std::max(t.ntile[KIND_X], ratio_tiles(N, P, t.xrows)) * sizeof(double);
     b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
     b += DWHIP_STAT_BLOCKS * 4 * sizeof(double) + 4096;
-    (void)M; (void)N; (void)P; (void)pM; (void)pN; (void)pP;
+    (void)M;
     return b;
 }
 
@@ -464,7 +515,12 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     } else if (rc != DWHIP_OK) {
         return rc;
     }
-    j->generic = !dwhip_fast_size_ok(w);
+    // the fused passes; else an extended job on them; else the any-size path
+    int64_t L[3] = {w[0], w[1], w[2]};  // transform lengths
+    j->ext = !dwhip_fast_size_ok(w) && j->allow_ext && dwhip_ext_size(w, pM, pN, pP, L);
+    j->generic = !j->ext && !dwhip_fast_size_ok(w);
+    if (!j->ext)
+        for (int d = 0; d < 3; ++d) L[d] = w[d];
     if (M * N * P > (int64_t)1 << 31 || w[0] * w[1] * w[2] > (int64_t)1 << 34) return DWHIP_ERR_SIZE;
     for (int d = 0; d < 3; ++d) {
         j->work[d] = w[d];
@@ -473,9 +529,14 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     const int niter = std::max(1, prm->iter_type == DWHIP_ITER_FIXED ? prm->niter : prm->maxiter);
 
     JobDev& d = j->d;
-    d.nx = (int)w[0];
-    d.ny = (int)w[1];
-    d.nz = (int)w[2];
+    d.nx = (int)L[0];
+    d.ny = (int)L[1];
+    d.nz = (int)L[2];
+    d.dx = (int)w[0];
+    d.ux = j->ext ? (int)round_up(w[0], 2) : (int)w[0];
+    d.uy = (int)w[1];
+    d.uz = (int)w[2];
+    d.ext = j->ext ? 1 : 0;
     d.h = d.nx / 2;
     d.hc = d.h + 1;
     d.hcs = (int)round_up(d.hc, 16);  // rows start on 128-byte lines
@@ -486,14 +547,24 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     // else the rule planner's
     DwhipPlanChoice cached;
     const DwhipPlanChoice* pc = j->force_plan;
-    if (!pc && !j->generic && dwhip_plan_cached(w, &cached)) pc = &cached;
-    dwhip_tile_config(w, &j->tiles, pc);
+    if (!pc && !j->generic && dwhip_plan_cached(L, &cached)) pc = &cached;
+    dwhip_tile_config(L, &j->tiles, pc);
+    if (j->ext) {
+        // C holds the data's planes, x tiles stay within a plane of data rows;
+        // the OTF's set-up walks the whole transform
+        DwhipTiles& t = j->tiles;
+        j->otf_tiles[0] = t.ntile[KIND_X];
+        j->otf_tiles[1] = t.ntile[KIND_Y];
+        j->otf_tiles[2] = t.ntile[KIND_Z];
+        t.ntile[KIND_X] = t.ntile[KIND_XR] = ratio_tiles(d.uy, d.uz, t.xrows);
+        t.ntile[KIND_Y] = t.ntile[KIND_Y] / d.nz * d.uz;
+    }
     {
         // pass D transforms slabs z < P; pass F too, except for RL, whose
         // ratio is 1e-6 outside the image
         const int nct = (d.hc + j->tiles.ycols - 1) / j->tiles.ycols;
         j->tiles.ntile[KIND_YD] = nct * (int)P;
-        j->tiles.ntile[KIND_YF] = prm->method == DWHIP_METHOD_RL ? nct * (int)w[2] : nct * (int)P;
+        j->tiles.ntile[KIND_YF] = prm->method == DWHIP_METHOD_RL ? nct * d.uz : nct * (int)P;
         // pass E: rows y < N of planes z < P for SHB (whose ratio is 0
         // elsewhere), all rows for RL
         if (prm->method != DWHIP_METHOD_RL) j->tiles.ntile[KIND_XR] = ratio_tiles(N, P, j->tiles.xrows);
@@ -531,20 +602,20 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
         const size_t V = (size_t)d.nx * d.ny * d.nz;
         size_t off = 0;
         auto take = [&](size_t bytes) { size_t o = off; off = round_up(off + bytes, 256); return o; };
-        DwhipLayout& L = j->lay;
+        DwhipLayout& lay = j->lay;
         const size_t Vh = (size_t)d.hcs * d.ny * d.nz;
-        L.C = take(Vh * sizeof(float2));
-        L.K = take(Vh * sizeof(float2));
-        L.U0 = take(V * sizeof(float));
-        L.U1 = take(V * sizeof(float));
-        L.W = d.has_w ? take(V * sizeof(float)) : 0;
-        L.part = take((size_t)d.ntile[KIND_XR] * sizeof(double));
-        L.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
-        L.err = take((size_t)niter * sizeof(float));
-        L.errd = take((size_t)niter * sizeof(double));
-        L.tw = take(j->tw.size() * sizeof(float2));
-        L.st = take(sizeof(JobState));
-        L.tab = take(64 + round_up(sizeof(JobDev), 64) + sizeof(GenDev));
+        lay.C = take(Vh * sizeof(float2));
+        lay.K = take(Vh * sizeof(float2));
+        lay.U0 = take(V * sizeof(float));
+        lay.U1 = take(V * sizeof(float));
+        lay.W = d.has_w ? take(V * sizeof(float)) : 0;
+        lay.part = take((size_t)d.ntile[KIND_XR] * sizeof(double));
+        lay.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
+        lay.err = take((size_t)niter * sizeof(float));
+        lay.errd = take((size_t)niter * sizeof(double));
+        lay.tw = take(j->tw.size() * sizeof(float2));
+        lay.st = take(sizeof(JobState));
+        lay.tab = take(64 + round_up(sizeof(JobDev), 64) + sizeof(GenDev));
         j->bytes = off;
         return DWHIP_OK;
     }
@@ -561,23 +632,24 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     }
 
     // layout of the job's block
-    const size_t V = (size_t)d.nx * d.ny * d.nz;
-    const size_t Vc = (size_t)d.hcs * d.ny * d.nz;
+    const size_t V = (size_t)d.ux * d.uy * d.uz;
+    const size_t Vc = (size_t)d.hcs * d.ny * d.uz;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off = round_up(off + bytes, 256); return o; };
-    DwhipLayout& L = j->lay;
-    L.C = take(Vc * sizeof(float2));
-    L.K = take(Vc * sizeof(float2));
-    L.U0 = take(V * sizeof(float));
-    L.U1 = take(V * sizeof(float));
-    L.W = d.has_w ? take(V * sizeof(float)) : 0;
-    L.part = take((size_t)std::max(d.ntile[KIND_X], d.ntile[KIND_XR]) * sizeof(double));
-    L.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
-    L.err = take((size_t)niter * sizeof(float));
-    L.errd = take((size_t)niter * sizeof(double));
-    L.tw = take(tw.size() * sizeof(float2));
-    L.st = take(sizeof(JobState));
-    L.tab = take(sizeof(BatchDev) + 64 + sizeof(JobDev));
+    DwhipLayout& lay = j->lay;
+    lay.C = take(Vc * sizeof(float2));
+    lay.K = take((size_t)d.hcs * d.ny * d.nz * sizeof(float2));
+    lay.U0 = take(V * sizeof(float));
+    lay.U1 = take(V * sizeof(float));
+    lay.W = d.has_w ? take(V * sizeof(float)) : 0;
+    lay.part = take((size_t)std::max(d.ntile[KIND_X], d.ntile[KIND_XR]) * sizeof(double));
+    lay.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
+    lay.err = take((size_t)niter * sizeof(float));
+    lay.errd = take((size_t)niter * sizeof(double));
+    lay.tw = take(tw.size() * sizeof(float2));
+    lay.st = take(sizeof(JobState));
+    lay.tab = take(sizeof(BatchDev) + 64 + sizeof(JobDev));
+    lay.otab = j->ext ? take(sizeof(BatchDev) + 64 + sizeof(JobDev)) : 0;
     j->bytes = off;
     return DWHIP_OK;
 }
@@ -615,6 +687,20 @@ int dwhip_job_bind(DwhipJob* j, void* mem, hipStream_t s)
     HIPCHK(hipMemcpyAsync(base + L.tw, j->tw.data(), j->tw.size() * sizeof(float2), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(j->bd, &j->bh, sizeof(j->bh), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(j->jd, &j->dcopy, sizeof(j->dcopy), hipMemcpyHostToDevice, s));
+    if (j->ext) {
+        // the OTF's set-up as a plain job of the transform's size, in K
+        j->obd = (BatchDev*)(base + L.otab);
+        j->ojd = (JobDev*)(base + L.otab + 64);
+        j->obh = j->bh;
+        j->odcopy = d;
+        JobDev& o = j->odcopy;
+        o.C = o.K;
+        o.ext = 0;
+        const int kinds[3] = {KIND_X, KIND_Y, KIND_Z};
+        for (int k = 0; k < 3; ++k) j->obh.ntile[kinds[k]] = o.ntile[kinds[k]] = j->otf_tiles[k];
+        HIPCHK(hipMemcpyAsync(j->obd, &j->obh, sizeof(j->obh), hipMemcpyHostToDevice, s));
+        HIPCHK(hipMemcpyAsync(j->ojd, &j->odcopy, sizeof(j->odcopy), hipMemcpyHostToDevice, s));
+    }
     if (j->generic) return dwhip_generic_bind(j, base + L.tab + 64 + round_up(sizeof(JobDev), 64), s);
     return DWHIP_OK;
 }
@@ -628,6 +714,14 @@ int dwhip_job_create(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int
     if (rc != DWHIP_OK) return rc;
     void* mem = nullptr;
     hipError_t e = job_mem_acquire(j->bytes, &mem);
+    if (e == hipErrorOutOfMemory && j->ext) {
+        // the any-size path needs less (no padded spectra)
+        (void)hipGetLastError();
+        j->allow_ext = false;
+        rc = dwhip_job_plan(j, im_dev, M, N, P, psf_dev, pM, pN, pP, prm, start_dev);
+        if (rc != DWHIP_OK) return rc;
+        e = job_mem_acquire(j->bytes, &mem);
+    }
     if (e != hipSuccess) return e == hipErrorOutOfMemory ? DWHIP_ERR_NOMEM : DWHIP_ERR_HIP;
     rc = dwhip_job_bind(j, mem, nullptr);
     if (rc == DWHIP_OK) {
@@ -644,30 +738,34 @@ int dwhip_job_create(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int
 double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
 {
     const double row = (double)d.hc * sizeof(float2);          // one complex x-row
-    const double Vc = row * d.ny * d.nz;
-    const double V = (double)d.nx * d.ny * d.nz * sizeof(float);
+    const double Kc = row * d.ny * d.nz;                       // the OTF
+    const double Vc = row * d.ny * d.uz;                       // one spectrum (its data planes)
+    const double Xc = row * d.uy * d.uz;                       // the x-rows of one (its data rows)
+    const double V = (double)d.dx * d.uy * d.uz * sizeof(float);
     const double img = (double)d.M * d.N * d.P * sizeof(float);
     const double slabP = row * d.ny * d.P;                     // z < P
     const double imgrows = row * d.N * d.P;                    // y < N, z < P
     if (!xkind) {
         switch (mode) {
-        case CM_ZCONV: return Vc + Vc + slabP;                 // read C, K; write z < P
-        case CM_ZCONVJ: return d.rl ? 3 * Vc : slabP + Vc + Vc; // read z < P (RL: all), K; write C
+        case CM_ZCONV: return Vc + Kc + slabP;                 // read C, K; write z < P
+        case CM_ZCONVJ: return (d.rl ? Vc : slabP) + Kc + Vc;  // read z < P (RL: all), K; write C
         case CM_YINV_IMG: return slabP + imgrows;              // slabs z < P, write y < N
-        case CM_YFWD_IMG: return d.rl ? 2 * Vc : imgrows + slabP;
+        case CM_YFWD_IMG: return d.rl ? Xc + Vc : imgrows + slabP;
+        case CM_YFWD:
+        case CM_YINV: return Xc + Vc;
         default: return 2 * Vc;
         }
     }
     switch (mode) {
-    case XM_PSF: return Vc + (double)d.pM * d.pN * d.pP * sizeof(float);
-    case XM_ONES: return Vc;
-    case XM_WEIGHTS: return Vc + V;
+    case XM_PSF: return Kc + (double)d.pM * d.pN * d.pP * sizeof(float);
+    case XM_ONES: return Xc;
+    case XM_WEIGHTS: return Xc + V;
     case XM_UPDATE:
         // SHB reads x_{k-1}, x_{k-2} (and W), writes x_k; RL reads x_{k-1}
         // (and W), writes x_k
-        if (iter == 0) return (d.rl ? 1 : 2) * V + Vc;
-        return 2 * Vc + ((d.rl ? 2 : 3) + (d.has_w ? 1 : 0)) * V;
-    case XM_RATIO: return d.rl ? imgrows + Vc + img : 2 * imgrows + img;
+        if (iter == 0) return (d.rl ? 1 : 2) * V + Xc;
+        return 2 * Xc + ((d.rl ? 2 : 3) + (d.has_w ? 1 : 0)) * V;
+    case XM_RATIO: return d.rl ? imgrows + Xc + img : 2 * imgrows + img;
     case XM_LOAD: return Vc + V;
     case XM_STORE: return Vc + V;
     default: return 0;
@@ -684,7 +782,7 @@ int dwhip_pass_x(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 {
     if (ntile <= 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    hipError_t e = dwhip_launch_xpass(mode, bd, jd, ntile, lds, s);
+    hipError_t e = dwhip_launch_xpass(mode, j->ext && bd != j->obd, bd, jd, ntile, lds, s);
     if (slot >= 0) dwhip_prof_end(s, slot, mode, dwhip_pass_bytes(1, mode, j->d, (int)host_iter(j, mode)));
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "x pass", __LINE__);
 }
@@ -694,7 +792,7 @@ int dwhip_pass_c(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 {
     if (ntile <= 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    hipError_t e = dwhip_launch_colpass(mode, bd, jd, ntile, lds, s);
+    hipError_t e = dwhip_launch_colpass(mode, j->ext && bd != j->obd, bd, jd, ntile, lds, s);
     if (slot >= 0) dwhip_prof_end(s, slot, 7 + mode, dwhip_pass_bytes(0, mode, j->d, 0));
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "column pass", __LINE__);
 }
@@ -714,13 +812,21 @@ int dwhip_job_setup(const DwhipJob* j, hipStream_t s)
     HIPCHK(dwhip_launch_stats(j->jd, 0, nblk, s));
     HIPCHK(dwhip_launch_start(j->jd, 0, 1024, s));
     // OTF: shifted PSF -> R2C -> K / (nx*ny*nz)
-    RCHK(dwhip_pass_x(XM_PSF, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
-    RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
-    RCHK(dwhip_pass_c(CM_ZOTF, j, j->bd, j->jd, t.ntile[KIND_Z], t.lds[KIND_Z], s));
+    {
+        const BatchDev* bd = j->ext ? j->obd : j->bd;
+        const JobDev* jd = j->ext ? j->ojd : j->jd;
+        RCHK(dwhip_pass_x(XM_PSF, j, bd, jd, j->ext ? j->otf_tiles[0] : t.ntile[KIND_X], t.lds[KIND_X], s));
+        RCHK(dwhip_pass_c(CM_YFWD, j, bd, jd, j->ext ? j->otf_tiles[1] : t.ntile[KIND_Y], t.lds[KIND_Y], s));
+        RCHK(dwhip_pass_c(CM_ZOTF, j, bd, jd, j->ext ? j->otf_tiles[2] : t.ntile[KIND_Z], t.lds[KIND_Z], s));
+    }
     if (j->d.has_w) {
         // P1 = IFFT(conj(K) FFT(1_box)); W = P1 > 0.01 ? 1/P1 : 0
         RCHK(dwhip_pass_x(XM_ONES, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
-        RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
+        // (an extended job continues the box as the adjoint reads it)
+        if (j->ext)
+            RCHK(dwhip_pass_c(CM_YFWD_IMG, j, j->bd, j->jd, t.ntile[KIND_YF], t.lds[KIND_YF], s));
+        else
+            RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
         RCHK(dwhip_pass_c(CM_ZCONVJ, j, j->bd, j->jd, t.ntile[KIND_Z], t.lds[KIND_Z], s));
         RCHK(dwhip_pass_c(CM_YINV, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
         RCHK(dwhip_pass_x(XM_WEIGHTS, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
@@ -875,13 +981,14 @@ static int hooked_loop(DwhipJob* job, const dwhip_params* prm, float* out, hipSt
         error = ek;
     }
     if (prm->hook_full) {
-        const int64_t w[3] = {d.nx, d.ny, d.nz};
+        const int64_t w[3] = {d.dx, d.uy, d.uz};
         const size_t V = (size_t)w[0] * w[1] * w[2];
         std::vector<float> full(V);
         if (job->d.rl && *nrun > 0) RCHK(dwhip_job_final_update(job, job->bd, job->jd, s));
         const int k = dwhip_result_iterate(job->d.rl != 0, *nrun);
         const float* U = (k & 1) ? d.U1 : d.U0;
-        HIPCHK(hipMemcpyAsync(full.data(), U, V * sizeof(float), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpy2DAsync(full.data(), w[0] * sizeof(float), U, d.ux * sizeof(float), w[0] * sizeof(float),
+                                (size_t)w[1] * w[2], hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         prm->hook(prm->hook_user, -1, 0.f, full.data(), w[0], w[1], w[2]);
         std::vector<float> hp((size_t)d.pM * d.pN * d.pP);
@@ -912,6 +1019,11 @@ static int run_job(const float* im, int64_t M, int64_t N, int64_t P, const float
     }
     if (mem) {
         rc = dwhip_job_plan(&job, im, M, N, P, psf, pM, pN, pP, prm, start);
+        if (rc == DWHIP_OK && job.bytes > cap && job.ext) {
+            // the any-size path needs less (no padded spectra)
+            job.allow_ext = false;
+            rc = dwhip_job_plan(&job, im, M, N, P, psf, pM, pN, pP, prm, start);
+        }
         if (rc == DWHIP_OK && job.bytes > cap) rc = DWHIP_ERR_SCRATCH;
         if (rc == DWHIP_OK) rc = dwhip_job_bind(&job, mem, s);
         if (rc != DWHIP_OK) {

@@ -29,7 +29,7 @@ struct DwhipPlanChoice {
 
 // Byte offsets of a job's buffers inside its device block.
 struct DwhipLayout {
-    size_t C, K, U0, U1, W, part, stat, err, errd, tw, st, tab;
+    size_t C, K, U0, U1, W, part, stat, err, errd, tw, st, tab, otab;
 };
 
 // One job: host copy of its descriptor plus its device block, which also
@@ -49,6 +49,15 @@ struct DwhipJob {
     size_t rtw_off = 0;
     BatchDev bh;              // host copies of the one-job table being uploaded
     JobDev dcopy;
+    // extended job (dwhip_ext_size): its OTF set-up runs the plain passes on a
+    // table of its own, with the transform's sizes and K in C's place
+    bool ext = false;
+    bool allow_ext = true;         // false: plan on the any-size path
+    int otf_tiles[3] = {0, 0, 0};  // x, y and z tiles of that set-up
+    BatchDev* obd = nullptr;
+    JobDev* ojd = nullptr;
+    BatchDev obh;
+    JobDev odcopy;
     // any-size path (generic.cpp): per-axis FFTs of any length; C holds
     // the work volume Z (half spectra, or real rows in place), K the OTF
     bool generic = false;
@@ -95,6 +104,8 @@ int dwhip_pass_c(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 void dwhip_job_free(DwhipJob* j);
 int dwhip_job_setup(const DwhipJob* j, hipStream_t s);
 int dwhip_job_round(DwhipJob* j, bool full, hipStream_t s);
+// whether the job runs its own passes one job at a time (in no batch)
+inline bool dwhip_job_solo(const DwhipJob* j) { return j->generic || j->ext; }
 int dwhip_job_final_update(DwhipJob* j, const BatchDev* bd, const JobDev* jd, hipStream_t s);
 // The per-image method on device pointers; mem/cap: the job's device block
 // when the caller provides it (nothing allocated then), nullptr to allocate.
@@ -113,6 +124,7 @@ int dwhip_capture(int (*body)(void* ctx, hipStream_t cs), void* ctx, hipGraphExe
 // any-size path (generic.cpp)
 bool dwhip_generic_size_ok(const int64_t* w);
 bool dwhip_fast_size_ok(const int64_t* w);
+bool dwhip_ext_size(const int64_t* w, int64_t pM, int64_t pN, int64_t pP, int64_t* L);
 int dwhip_generic_plan(DwhipJob* j);
 int dwhip_generic_bind(DwhipJob* j, char* gdev, hipStream_t s);
 int dwhip_generic_setup(const DwhipJob* j, hipStream_t s);

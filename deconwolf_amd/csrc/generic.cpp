@@ -1,7 +1,8 @@
 // Host side of the any-size path (generic_dev.h, k_generic.hip): plans,
 // twiddle and Bluestein tables, the job layout, and the set-up, round and
 // final-update sequences that the per-image driver (dwhip.cpp) runs for a
-// job whose work size the fused passes cannot transform.
+// job whose work size neither the fused passes nor an extended job on them
+// (dwhip_ext_size) transform.
 #include <hip/hip_runtime.h>
 
 #include <math.h>

@@ -7,14 +7,22 @@
 #define DWHIP_CAT2(a, b) a##b
 #define DWHIP_CAT(a, b) DWHIP_CAT2(a, b)
 
-extern "C" hipError_t DWHIP_CAT(dwhip_launch_c, CMODE)(const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+#ifdef PASS_EXT  // the mode's kernel for extended jobs
+#define PASS_LAUNCH DWHIP_CAT(dwhip_launch_ce, CMODE)
+#define PASS_EXT_V true
+#else
+#define PASS_LAUNCH DWHIP_CAT(dwhip_launch_c, CMODE)
+#define PASS_EXT_V false
+#endif
+
+extern "C" hipError_t PASS_LAUNCH(const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
                                                       hipStream_t s)
 {
     static bool once = false;
     if (!once) {
         once = true;
-        dwhip_allow_big_lds(reinterpret_cast<const void*>(k_colpass<CMODE>));
+        dwhip_allow_big_lds(reinterpret_cast<const void*>(k_colpass<CMODE, PASS_EXT_V>));
     }
-    hipLaunchKernelGGL(k_colpass<CMODE>, dim3(grid), dim3(col_threads<CMODE>()), lds, s, bd, jobs);
+    hipLaunchKernelGGL((k_colpass<CMODE, PASS_EXT_V>), dim3(grid), dim3(col_threads<CMODE>()), lds, s, bd, jobs);
     return hipGetLastError();
 }

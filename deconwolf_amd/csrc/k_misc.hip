@@ -122,15 +122,15 @@ __global__ __launch_bounds__(STHR) void k_stats_final(const JobDev* __restrict__
 __global__ __launch_bounds__(STHR) void k_start(const JobDev* __restrict__ jobs, int j)
 {
     const JobDev& J = jobs[j];
-    const size_t n = (size_t)J.nx * J.ny * J.nz;
+    const size_t n = (size_t)J.ux * J.uy * J.uz;
     const float c0 = J.st->c0;
     const float* src = J.start_img ? J.start_img : J.im;
     for (size_t i = (size_t)blockIdx.x * STHR + threadIdx.x; i < n; i += (size_t)gridDim.x * STHR) {
         float v = c0;
         if (J.start_identity) {
-            const int m = (int)(i % J.nx);
-            const size_t r = i / J.nx;
-            const int yy = (int)(r % J.ny), zz = (int)(r / J.ny);
+            const int m = (int)(i % J.ux);
+            const size_t r = i / J.ux;
+            const int yy = (int)(r % J.uy), zz = (int)(r / J.uy);
             v = (m < J.M && yy < J.N && zz < J.P) ? src[m + (size_t)J.M * (yy + (size_t)J.N * zz)] : 0.f;
         }
         J.U0[i] = v;
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(STHR) void k_crop(const JobDev* __restrict__ jobs, 
     const int nrows = J.N * J.P;
     for (int r = blockIdx.x; r < nrows; r += gridDim.x) {
         const int zz = r / J.N, yy = r - zz * J.N;
-        const float* src = U + (size_t)J.nx * (yy + (size_t)J.ny * zz);
+        const float* src = U + (size_t)J.ux * (yy + (size_t)J.uy * zz);
         float* dst = out + (size_t)J.M * r;
         for (int m = threadIdx.x; m < J.M; m += STHR) dst[m] = src[m];
     }
@@ -218,6 +218,10 @@ DECL_LAUNCH(dwhip_launch_x3)
 DECL_LAUNCH(dwhip_launch_x4)
 DECL_LAUNCH(dwhip_launch_x5)
 DECL_LAUNCH(dwhip_launch_x6)
+DECL_LAUNCH(dwhip_launch_xe1)
+DECL_LAUNCH(dwhip_launch_xe2)
+DECL_LAUNCH(dwhip_launch_xe3)
+DECL_LAUNCH(dwhip_launch_xe4)
 DECL_LAUNCH(dwhip_launch_c0)
 DECL_LAUNCH(dwhip_launch_c1)
 DECL_LAUNCH(dwhip_launch_c2)
@@ -227,39 +231,40 @@ DECL_LAUNCH(dwhip_launch_c5)
 DECL_LAUNCH(dwhip_launch_c6)
 DECL_LAUNCH(dwhip_launch_c7)
 DECL_LAUNCH(dwhip_launch_c8)
+DECL_LAUNCH(dwhip_launch_ce0)
+DECL_LAUNCH(dwhip_launch_ce1)
+DECL_LAUNCH(dwhip_launch_ce3)
+DECL_LAUNCH(dwhip_launch_ce4)
+DECL_LAUNCH(dwhip_launch_ce7)
+DECL_LAUNCH(dwhip_launch_ce8)
 
 extern "C" {
 
-hipError_t dwhip_launch_xpass(int mode, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s)
+typedef hipError_t (*pass_launch)(const BatchDev*, const JobDev*, int, size_t, hipStream_t);
+
+hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+                              hipStream_t s)
 {
     static_assert(XM_PSF == 0 && XM_STORE == 6, "X modes 0..6");
-    switch (mode) {
-    case 0: return dwhip_launch_x0(bd, jobs, grid, lds, s);
-    case 1: return dwhip_launch_x1(bd, jobs, grid, lds, s);
-    case 2: return dwhip_launch_x2(bd, jobs, grid, lds, s);
-    case 3: return dwhip_launch_x3(bd, jobs, grid, lds, s);
-    case 4: return dwhip_launch_x4(bd, jobs, grid, lds, s);
-    case 5: return dwhip_launch_x5(bd, jobs, grid, lds, s);
-    case 6: return dwhip_launch_x6(bd, jobs, grid, lds, s);
-    default: return hipErrorInvalidValue;
-    }
+    static const pass_launch f[2][7] = {
+        {dwhip_launch_x0, dwhip_launch_x1, dwhip_launch_x2, dwhip_launch_x3, dwhip_launch_x4, dwhip_launch_x5,
+         dwhip_launch_x6},
+        {nullptr, dwhip_launch_xe1, dwhip_launch_xe2, dwhip_launch_xe3, dwhip_launch_xe4, nullptr, nullptr}};
+    if (mode < 0 || mode > 6 || !f[ext ? 1 : 0][mode]) return hipErrorInvalidValue;
+    return f[ext ? 1 : 0][mode](bd, jobs, grid, lds, s);
 }
 
-hipError_t dwhip_launch_colpass(int mode, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s)
+hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+                                hipStream_t s)
 {
     static_assert(CM_YFWD == 0 && CM_YFWD_IMG == 8 && DWHIP_N_CMODES == 9, "column modes 0..8");
-    switch (mode) {
-    case 0: return dwhip_launch_c0(bd, jobs, grid, lds, s);
-    case 1: return dwhip_launch_c1(bd, jobs, grid, lds, s);
-    case 2: return dwhip_launch_c2(bd, jobs, grid, lds, s);
-    case 3: return dwhip_launch_c3(bd, jobs, grid, lds, s);
-    case 4: return dwhip_launch_c4(bd, jobs, grid, lds, s);
-    case 5: return dwhip_launch_c5(bd, jobs, grid, lds, s);
-    case 6: return dwhip_launch_c6(bd, jobs, grid, lds, s);
-    case 7: return dwhip_launch_c7(bd, jobs, grid, lds, s);
-    case 8: return dwhip_launch_c8(bd, jobs, grid, lds, s);
-    default: return hipErrorInvalidValue;
-    }
+    static const pass_launch f[2][DWHIP_N_CMODES] = {
+        {dwhip_launch_c0, dwhip_launch_c1, dwhip_launch_c2, dwhip_launch_c3, dwhip_launch_c4, dwhip_launch_c5,
+         dwhip_launch_c6, dwhip_launch_c7, dwhip_launch_c8},
+        {dwhip_launch_ce0, dwhip_launch_ce1, nullptr, dwhip_launch_ce3, dwhip_launch_ce4, nullptr, nullptr,
+         dwhip_launch_ce7, dwhip_launch_ce8}};
+    if (mode < 0 || mode >= DWHIP_N_CMODES || !f[ext ? 1 : 0][mode]) return hipErrorInvalidValue;
+    return f[ext ? 1 : 0][mode](bd, jobs, grid, lds, s);
 }
 
 hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int nblk, hipStream_t s)

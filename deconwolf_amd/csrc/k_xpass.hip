@@ -28,14 +28,22 @@
 #define DWHIP_CAT2(a, b) a##b
 #define DWHIP_CAT(a, b) DWHIP_CAT2(a, b)
 
-extern "C" hipError_t DWHIP_CAT(dwhip_launch_x, XMODE)(const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+#ifdef PASS_EXT  // the mode's kernel for extended jobs
+#define PASS_LAUNCH DWHIP_CAT(dwhip_launch_xe, XMODE)
+#define PASS_EXT_V true
+#else
+#define PASS_LAUNCH DWHIP_CAT(dwhip_launch_x, XMODE)
+#define PASS_EXT_V false
+#endif
+
+extern "C" hipError_t PASS_LAUNCH(const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
                                                       hipStream_t s)
 {
     static bool once = false;
     if (!once) {
         once = true;
-        dwhip_allow_big_lds(reinterpret_cast<const void*>(k_xpass<XMODE>));
+        dwhip_allow_big_lds(reinterpret_cast<const void*>(k_xpass<XMODE, PASS_EXT_V>));
     }
-    hipLaunchKernelGGL(k_xpass<XMODE>, dim3(grid), dim3(XTHR), lds, s, bd, jobs);
+    hipLaunchKernelGGL((k_xpass<XMODE, PASS_EXT_V>), dim3(grid), dim3(XTHR), lds, s, bd, jobs);
     return hipGetLastError();
 }

@@ -39,6 +39,14 @@ struct JobState {
 struct JobDev {
     // transform (work) size; h = nx/2, hc = h+1 complex per x-row, hcs = row stride
     int nx, ny, nz, h, hc, hcs;
+    // the real volumes U0, U1 and W: ux x uy x uz values, of which dx along x
+    // hold data (ux = dx rounded up to even in an extended job, else ux = dx =
+    // nx, uy = ny, uz = nz)
+    int dx, ux, uy, uz;
+    // 1: extended job (the EXT kernels): the convolution has period dx, uy, uz
+    // but is transformed at nx, ny, nz, the data of every axis that is longer
+    // in the transform continued periodically as far as the PSF reaches
+    int ext;
     // image and PSF sizes
     int M, N, P;
     int pM, pN, pP;
@@ -68,11 +76,11 @@ struct JobDev {
     float bg_user;
     JobState* st;       // device-written state of this job
     // buffers
-    float2* C;          // complex work volume, [nz][ny][hcs]
+    float2* C;          // complex work volume, [uz][ny][hcs]
     float2* K;          // OTF / (nx*ny*nz), [nz][ny][hcs]
     float* U0;          // x_k lives in U[k & 1]
     float* U1;
-    float* W;           // Bertero weights, nx*ny*nz (unused when has_w == 0)
+    float* W;           // Bertero weights, ux*uy*uz (unused when has_w == 0)
     const float* im;    // image M*N*P (offset already added)
     const float* psf;   // PSF pM*pN*pP
     const float* start_img;  // M*N*P start image for identity/LP starts

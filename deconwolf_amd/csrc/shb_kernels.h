@@ -15,6 +15,17 @@ enum { XM_PSF = 0, XM_ONES = 1, XM_WEIGHTS = 2, XM_UPDATE = 3, XM_RATIO = 4, XM_
 enum { CM_YFWD = 0, CM_YINV = 1, CM_ZOTF = 2, CM_ZCONV = 3, CM_ZCONVJ = 4, CM_ZFWD = 5, CM_ZINV = 6,
        CM_YINV_IMG = 7, CM_YFWD_IMG = 8 };
 #define DWHIP_N_CMODES 9
+// Passes an extended job runs (JobDev.ext): its OTF is set up by the plain
+// passes at the transform size, and its weights by YFWD_IMG (the ones box is
+// zero where that pass does not read).
+__host__ __device__ constexpr bool xmode_has_ext(int m)
+{
+    return m == XM_ONES || m == XM_WEIGHTS || m == XM_UPDATE || m == XM_RATIO;
+}
+__host__ __device__ constexpr bool cmode_has_ext(int m)
+{
+    return m == CM_YFWD || m == CM_YINV || m == CM_ZCONV || m == CM_ZCONVJ || m == CM_YINV_IMG || m == CM_YFWD_IMG;
+}
 __host__ __device__ constexpr bool cmode_is_y(int m)
 {
     return m == CM_YFWD || m == CM_YINV || m == CM_YINV_IMG || m == CM_YFWD_IMG;
@@ -60,8 +71,9 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #endif
 
 extern "C" {
-hipError_t dwhip_launch_xpass(int mode, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
-hipError_t dwhip_launch_colpass(int mode, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
+// ext: 1 launches the kernels of extended jobs (a table holds one kind)
+hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
+hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
 hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int nblk, hipStream_t s);
 hipError_t dwhip_launch_start(const JobDev* jobs, int j, int grid, hipStream_t s);
 hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int njobs, int advance, hipStream_t s);

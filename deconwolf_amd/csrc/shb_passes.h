@@ -68,6 +68,19 @@ __device__ __forceinline__ float shb_extrap(float x, float xp, double alpha, flo
     return p < bg ? bg : p;
 }
 
+// Extended jobs: a convolution of period n with a PSF of p values, its
+// maximum at mid, as one of length L >= n + p - 1.  Output i < n of the
+// forward model reads inputs i - (p - 1 - mid) .. i + mid, the adjoint's
+// i - mid .. i + (p - 1 - mid); so element e >= n of the input holds the
+// data's value e - n for the `right` values after the end and e - L + n for
+// those before the start (kept at the end of the transform); elements between
+// them reach no output that is read.
+__device__ __forceinline__ int ext_right(int mid, int p, bool adjoint) { return adjoint ? p - 1 - mid : mid; }
+__device__ __forceinline__ int ext_index(int e, int n, int L, int right)
+{
+    return e < n ? e : e < n + right ? e - n : max(e - L + n, 0);
+}
+
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* red)
 {
@@ -318,7 +331,11 @@ __device__ __forceinline__ void x_fft(const FftPlanDev& p, const StageGeo& g, in
 }
 
 // One X tile t of job J; FR1 > 0: the job's x plan is (FR1, FR2).
-template <int MODE, int FR1, int FR2>
+// EXT: an extended job.  Its tiles stay within one plane (C has ny rows per
+// plane, the real volumes uy), the elementwise step runs over the dx data
+// values of each row, and the row is continued periodically to the transform
+// length before the forward transform.
+template <int MODE, int FR1, int FR2, bool EXT>
 __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, float2* lds, double* red)
 {
     constexpr bool XNT = x_nt(MODE);
@@ -330,7 +347,17 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         const int ny = J.ny, hcs = J.hcs;
         int row0 = lt * J.xrows;
         int nrows = min(J.xrows, ny * J.nz - row0);
-        if (MODE == XM_RATIO && !J.rl) {
+        int urow0 = row0;  // the tile's first row in the real volumes
+        int ez = 0, ey0 = 0;
+        if (EXT) {
+            const int rows = (MODE == XM_RATIO && !J.rl) ? J.N : J.uy;
+            const int tpp = (rows + J.xrows - 1) / J.xrows;
+            ez = lt / tpp;
+            ey0 = (lt - ez * tpp) * J.xrows;
+            row0 = ez * ny + ey0;
+            urow0 = ez * J.uy + ey0;
+            nrows = min(J.xrows, rows - ey0);
+        } else if (MODE == XM_RATIO && !J.rl) {
             // the SHB ratio is 0 outside the image box and only y < N, z < P
             // rows of y are used: pass E's tiles cover exactly those rows,
             // ceil(N / xrows) tiles within each plane z < P (the RL ratio is
@@ -368,7 +395,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             uint64_t live = ~0ull;  // bit b: row row0 + b is transformed
             if (MODE == XM_RATIO) {
                 live = 0;
-                int z = row0 / ny, y = row0 - (row0 / ny) * ny;
+                int z = EXT ? ez : row0 / ny, y = EXT ? ey0 : row0 - (row0 / ny) * ny;
                 for (int b = 0; b < nrows; ++b) {
                     if (z < J.P && y < J.N) live |= 1ull << b;
                     if (++y == ny) { y = 0; ++z; }
@@ -410,8 +437,8 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             auto split_src = [&](int pen, int i) {
                 const int row = row0 + pen;
                 if (MODE == XM_RATIO) {
-                    const int zz = row / ny;
-                    if (zz >= J.P || row - zz * ny >= J.N) return make_float2(0.f, 0.f);
+                    const int zz = EXT ? ez : row / ny;
+                    if (zz >= J.P || (EXT ? ey0 + pen : row - zz * ny) >= J.N) return make_float2(0.f, 0.f);
                 }
                 // plain loads: each spectrum line is read twice (elements k
                 // and h - k), and a nontemporal hint on the first read drops
@@ -427,7 +454,12 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         // elementwise step on packed real pairs (elements 2n, 2n+1 of a row),
         // in natural order in LDS; loads of XCHUNK elements are issued together
         double acc = 0;
-        const int nwork = nrows * h;
+        // pairs per row (EXT: the data's), and pair w's place in LDS
+        const int dp = EXT ? J.ux >> 1 : h;
+        const int ux = EXT ? J.ux : nx;
+        const uint32_t dpmagic = EXT ? fdiv_magic((uint32_t)dp) : hmagic;
+        const int nwork = nrows * dp;
+        auto lix = [&](int w) { return EXT ? w + (int)fdiv((uint32_t)w, dpmagic) * (h - dp) : w; };
         DWHIP_GL float* Uk = gp((iter & 1) ? J.U1 : J.U0);          // x_{k-2} in, x_k out (k > 0)
         const DWHIP_GL float* Ukm1 = gp((iter & 1) ? J.U0 : J.U1);  // x_{k-1}
         DWHIP_GL float* U0 = gp(J.U0);
@@ -439,9 +471,9 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         const double al = MODE == XM_UPDATE ? shb_alpha(iter, J.alphamax) : 0.0;
         // the SHB ratio pass's tiles lie within one plane: its rows' y and z
         // come from the tile (no division per element)
-        const bool plane_tile = MODE == XM_RATIO && !J.rl;
-        const int tz = plane_tile ? row0 / ny : 0;
-        const int ty0 = plane_tile ? row0 - tz * ny : 0;
+        const bool plane_tile = EXT || (MODE == XM_RATIO && !J.rl);
+        const int tz = EXT ? ez : plane_tile ? row0 / ny : 0;
+        const int ty0 = EXT ? ey0 : plane_tile ? row0 - tz * ny : 0;
         // chunks of XCHUNK elements per thread; full chunks carry no bounds
         // tests, so their loads and arithmetic schedule as straight-line code
         auto chunk = [&](int w0, auto full) {
@@ -452,9 +484,9 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
 #pragma unroll
             for (int q = 0; q < XCHUNK; ++q) {
                 const int w = min(w0 + q * XTHR, nwork - 1);
-                const int bb = (int)fdiv((uint32_t)w, hmagic);
-                const int n = w - bb * h;
-                const int row = row0 + bb;
+                const int bb = (int)fdiv((uint32_t)w, dpmagic);
+                const int n = w - bb * dp;
+                const int row = urow0 + bb;
                 if (plane_tile) {
                     yy[q] = ty0 + bb;
                     zz[q] = tz;
@@ -463,13 +495,13 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                     zz[q] = row / ny;
                 }
                 m0[q] = 2 * n;
-                vi[q] = (size_t)row * nx + 2 * n;
+                vi[q] = (size_t)row * ux + 2 * n;
                 a[q] = b[q] = c[q] = wv[q] = make_float2(0.f, 0.f);
             }
 #pragma unroll
             for (int q = 0; q < XCHUNK; ++q) {
                 if (!FULL::value && w0 + q * XTHR >= nwork) continue;
-                if (inv) a[q] = lds[w0 + q * XTHR];
+                if (inv) a[q] = lds[lix(w0 + q * XTHR)];
                 if (MODE == XM_UPDATE) {
                     b[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Ukm1 + vi[q]));
                     if (!J.rl) c[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Uk + vi[q]));
@@ -592,7 +624,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                     }
                     out = make_float2(r[0], r[1]);
                 }
-                lds[w] = out;
+                lds[lix(w)] = out;
             }
                 };
         // job flags read once, before the element loops' stores (the
@@ -602,9 +634,9 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         const float lo = J.positivity ? bg : -INFINITY;  // x_k < lo -> lo (method_shb.c:366-374)
         if (DWHIP_X_FAST && MODE == XM_UPDATE && !rl && iter > 0) {
             // SHB iteration k > 0.  The tile's x-rows row0 .. row0+nrows-1
-            // are consecutive in every real volume (row stride nx = 2h), so
+            // are consecutive in every real volume (row stride 2 * dp), so
             // packed pair w of the tile is pair w from the tile's first voxel.
-            const size_t tb = (size_t)row0 * nx;
+            const size_t tb = (size_t)urow0 * ux;
             const DWHIP_GL float2* __restrict__ xm1 = reinterpret_cast<const DWHIP_GL float2*>(Ukm1 + tb);
             DWHIP_GL float2* __restrict__ xio = reinterpret_cast<DWHIP_GL float2*>(Uk + tb);  // x_{k-2} in, x_k out
             const DWHIP_GL float2* __restrict__ wt = reinterpret_cast<const DWHIP_GL float2*>(W + tb);
@@ -615,7 +647,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                 for (int q = 0; q < XCHUNK; ++q) {
                     const int w = w0 + q * XTHR;
                     if (!FULL && w >= nwork) continue;
-                    a[q] = lds[w];
+                    a[q] = lds[lix(w)];
                     b[q] = ldgs<DWHIP_NT_STATE>(xm1 + w);
                     c[q] = ldgs<DWHIP_NT_STATE>(xio + w);
                     wv[q] = HW ? ldgs<DWHIP_NT_STATE>(wt + w) : make_float2(1.f, 1.f);
@@ -632,7 +664,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                     xk.x = xk.x < lo ? lo : xk.x;
                     xk.y = xk.y < lo ? lo : xk.y;
                     stgs<DWHIP_NT_STATE>(xio + w, xk);
-                    lds[w] = make_float2(shb_extrap(xk.x, b[q].x, al, bg), shb_extrap(xk.y, b[q].y, al, bg));
+                    lds[lix(w)] = make_float2(shb_extrap(xk.x, b[q].x, al, bg), shb_extrap(xk.y, b[q].y, al, bg));
                 }
             };
             auto rows = [&](auto hw) {
@@ -644,7 +676,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                 rows(BoolC<true>());
             else
                 rows(BoolC<false>());
-        } else if (DWHIP_X_FAST && MODE == XM_RATIO && plane_tile && h > 1) {
+        } else if (DWHIP_X_FAST && MODE == XM_RATIO && !J.rl && dp > 1) {
             // SHB ratio over a plane tile: every row is an image row (y < N,
             // z < P); pair w holds columns 2n, 2n+1 of tile row w / h.  Image
             // loads are clamped into the tile's rows and dropped beyond
@@ -659,11 +691,11 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
 #pragma unroll
                 for (int q = 0; q < XCHUNK; ++q) {
                     const int w = FULL ? w0 + q * XTHR : min(w0 + q * XTHR, nwork - 1);
-                    const int bb = (int)__umulhi((uint32_t)w, hmagic);  // h > 1: hmagic is the magic of h
-                    const int n = w - bb * h;
+                    const int bb = (int)__umulhi((uint32_t)w, dpmagic);  // dp > 1: never the encoding of 1
+                    const int n = w - bb * dp;
                     m0[q] = 2 * n;
                     const int i0 = bb * M + 2 * n;
-                    a[q] = lds[w];
+                    a[q] = lds[EXT ? bb * h + n : w];
                     gv[q] = make_float2(imt[min(i0, ilast)], imt[min(i0 + 1, ilast)]);
                 }
 #pragma unroll
@@ -691,7 +723,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                         if (fabs(yd) < 1e-6) rv = g / (float)copysign(1e-6, yd);  // method_shb.c:41-42
                         r[e] = valid ? rv : 0.f;
                     }
-                    lds[w] = make_float2(r[0], r[1]);
+                    lds[lix(w)] = make_float2(r[0], r[1]);
                 }
             };
             auto rows = [&](auto idiv) {
@@ -713,6 +745,22 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             if (tid == 0) gp(J.part)[lt] = s;
         }
         __syncthreads();
+        if (EXT && fwd) {
+            // values dx .. nx-1 of each row: the data's period continued on
+            // both sides (see ext_index)
+            const int dx = J.dx, fill = nx - dx;
+            if (fill > 0) {
+                const int b = ext_right(st->mid[0], J.pM, MODE != XM_UPDATE);
+                const uint32_t fmagic = fdiv_magic((uint32_t)fill);
+                float* ldsf = reinterpret_cast<float*>(lds);
+                for (int w = tid; w < nrows * fill; w += XTHR) {
+                    const int r = (int)fdiv((uint32_t)w, fmagic);
+                    const int e = dx + (w - r * fill);
+                    ldsf[r * nx + e] = ldsf[r * nx + ext_index(e, dx, nx, b)];
+                }
+                __syncthreads();
+            }
+        }
 
         if (fwd) {
             x_fft<FR1, FR2, -1, true, true>(J.pxf, g, tid, lds, gp(J.tw), lds_src, lds_dst);
@@ -800,7 +848,7 @@ constexpr bool x_reversed()
     return (MODE == XM_UPDATE && DWHIP_REV_UPDATE) || (MODE == XM_RATIO && DWHIP_REV_RATIO);
 }
 
-template <int MODE>
+template <int MODE, bool EXT>
 __global__ __launch_bounds__(XTHR) DWHIP_X_OCC void k_xpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
 {
     extern __shared__ float2 lds[];
@@ -814,11 +862,11 @@ __global__ __launch_bounds__(XTHR) DWHIP_X_OCC void k_xpass(const BatchDev* __re
         if (J.dev_stop && gp(J.st)->stop) continue;  // the stopping rule ended this job
         if constexpr (x_fixed_mode(MODE)) {
             if (J.pxf.nst == 2 && J.pxf.radix[0] == 25 && J.pxf.radix[1] == 25) {
-                xpass_tile<MODE, 25, 25>(J, t, threadIdx.x, lds, red);
+                xpass_tile<MODE, 25, 25, EXT>(J, t, threadIdx.x, lds, red);
                 continue;
             }
         }
-        xpass_tile<MODE, 0, 0>(J, t, threadIdx.x, lds, red);
+        xpass_tile<MODE, 0, 0, EXT>(J, t, threadIdx.x, lds, red);
     }
 }
 
@@ -909,6 +957,28 @@ struct ColPencils {
     }
 };
 
+// Input pencils of an extended job: element i of the transform is the data's
+// value ext_index(i), zero from nv on (rows a pruned pass skips).
+template <bool NT>
+struct WrapPencils {
+    const DWHIP_GL float2* p;
+    size_t stride;
+    int npv, nv;
+    int n, L, right;  // period, transform length, values continued at the end
+    static constexpr bool kStrided = true;
+    __device__ __forceinline__ float2 operator()(int pen, int i) const
+    {
+        const int s = ext_index(i, n, L, right);
+        return (pen < npv && s < nv) ? ldgs<NT>(p + s * stride + pen) : make_float2(0.f, 0.f);
+    }
+    template <int R>
+    __device__ __forceinline__ void load(int pen, int j, int nb, float2* v) const
+    {
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = (*this)(pen, j + r * nb);
+    }
+};
+
 // Workgroup b runs on XCD b mod 8 (dispatch is round robin over the 8 XCDs,
 // each with its own L2).  Column tile t covers B adjacent kx columns, so
 // tiles t and t+1 share the 128-byte lines of a row when B*8 < 128: map
@@ -943,7 +1013,7 @@ constexpr int col_waves()
     return cmode_is_y(MODE) ? DWHIP_Y_WAVES : DWHIP_Z_WAVES;
 }
 
-template <int MODE>
+template <int MODE, bool EXT>
 __global__ __launch_bounds__(col_threads<MODE>()) __attribute__((amdgpu_waves_per_eu(col_waves<MODE>())))
 void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
 {
@@ -978,11 +1048,23 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         g.nthr = NT;
         g.npshift = __ffs(B) - 1;  // B is a power of two
         // elements read (i < nin) and written (i < nout) along the pencil
-        const int nin = (MODE == CM_YFWD_IMG && !J.rl) ? J.N : (MODE == CM_ZCONVJ && !J.rl) ? J.P : g.n;
-        const int nout = (MODE == CM_YINV_IMG) ? J.N : (MODE == CM_ZCONV) ? J.P : g.n;
+        const int nd = EXT ? (ykind ? J.uy : J.uz) : g.n;  // data values along the pencil
+        const int nin = (MODE == CM_YFWD_IMG && !J.rl) ? J.N : (MODE == CM_ZCONVJ && !J.rl) ? J.P
+                        : (MODE == CM_YINV || MODE == CM_YINV_IMG) ? g.n : nd;
+        const int nout = (MODE == CM_YINV_IMG) ? J.N : (MODE == CM_ZCONV) ? J.P
+                         : (MODE == CM_YINV || MODE == CM_ZCONVJ) ? nd : g.n;
 
         // (Z tiles only: the unmasked forms push 1024-thread Y tiles past 128 VGPRs)
-        const ColPencils<cnt> gsrc{gp(J.C) + off, stride, nb, nin, !ykind && nb == B && nin == g.n};
+        auto make_src = [&]() {
+            if constexpr (EXT && MODE != CM_YINV && MODE != CM_YINV_IMG) {
+                constexpr bool adjoint = MODE == CM_YFWD_IMG || MODE == CM_ZCONVJ;
+                const int right = ext_right(gp(J.st)->mid[ykind ? 1 : 2], ykind ? J.pN : J.pP, adjoint);
+                return WrapPencils<cnt>{gp(J.C) + off, stride, nb, nin, nd, g.n, right};
+            } else {
+                return ColPencils<cnt>{gp(J.C) + off, stride, nb, nin, !ykind && nb == B && nin == g.n};
+            }
+        };
+        const auto gsrc = make_src();
         const ColPencils<cnt> gdst{dst, stride, nb, nout, !ykind && nb == B && nout == g.n};
         if (MODE == CM_YFWD || MODE == CM_YFWD_IMG) {
             fft_tile<DWHIP_YMAXE, -1, true, DWHIP_RMAX_Y, false, false>(J.pyf, g, tid, lds, gp(J.tw), gsrc, gdst);
