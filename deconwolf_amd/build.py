@@ -59,7 +59,8 @@ def units():
     u.append(("k_bw.hip", [], "k_bw.o"))
     u.append(("noalloc.hip", [], "noalloc.o"))
     u.append(("k_generic.hip", [], "k_generic.o"))
-    for src in ("dwhip.cpp", "profile.cpp", "batch.cpp", "tiling.cpp", "graph.cpp", "generic.cpp", "tune.cpp"):
+    for src in ("dwhip.cpp", "profile.cpp", "batch.cpp", "tiling.cpp", "graph.cpp", "generic.cpp", "tune.cpp",
+                "transfer.cpp"):
         if os.path.exists(os.path.join(CSRC, src)):
             u.append((src, [], src.replace(".cpp", ".o")))
     return u

@@ -1187,13 +1187,15 @@ static int run_host(const float* im, int64_t M, int64_t N, int64_t P, const floa
     rc = dwhip_init();
     if (rc != DWHIP_OK) return rc;
     const bool has_start = prm->start != DWHIP_START_FLAT && prm->start_image;
-    float *dim = nullptr, *dpsf = nullptr, *dout = nullptr, *dstart = nullptr;
+    // one block: the image, the result, the PSF and the start image
+    const size_t o_out = round_up(n * sizeof(float), 256), o_psf = 2 * o_out;
+    const size_t o_start = o_psf + round_up(np * sizeof(float), 256);
+    char* block = nullptr;
     hipStream_t s = nullptr;
     hipError_t e = hipStreamCreate(&s);
-    if (e == hipSuccess) e = hipMalloc(&dim, n * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&dpsf, np * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&dout, n * sizeof(float));
-    if (e == hipSuccess && has_start) e = hipMalloc(&dstart, n * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&block, o_start + (has_start ? n * sizeof(float) : 0));
+    float *dim = (float*)block, *dpsf = (float*)(block + o_psf), *dout = (float*)(block + o_out);
+    float* dstart = has_start ? (float*)(block + o_start) : nullptr;
     if (e == hipSuccess) e = hipMemcpy(dim, im, n * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(dpsf, psf, np * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess && has_start) e = hipMemcpy(dstart, prm->start_image, n * sizeof(float), hipMemcpyHostToDevice);
@@ -1204,14 +1206,10 @@ static int run_host(const float* im, int64_t M, int64_t N, int64_t P, const floa
         p2.start_image = dstart;
         rc = run_job(dim, M, N, P, dpsf, pM, pN, pP, &p2, dout, st, s, nullptr, 0);
         if (rc == DWHIP_OK) {
-            e = hipMemcpy(out, dout, n * sizeof(float), hipMemcpyDeviceToHost);
-            if (e != hipSuccess) rc = dwhip_hip_fail(e, "download", __LINE__);
+            rc = dwhip_download(out, dout, n * sizeof(float), s);
         }
     }
-    if (dim) hipFree(dim);
-    if (dpsf) hipFree(dpsf);
-    if (dout) hipFree(dout);
-    if (dstart) hipFree(dstart);
+    if (block) hipFree(block);
     if (s) hipStreamDestroy(s);
     return rc;
 }

@@ -293,7 +293,10 @@ def fim_normalize_sum1(psf):
     """psf / sum(psf), sum in double (src/fim.c:900-912)."""
     psf = np.asarray(psf, dtype=np.float32)
     s = float(np.sum(psf, dtype=np.float64))
-    return (psf.astype(np.float64) / s).astype(np.float32)
+    # the double quotient rounded to float, without double temporaries
+    out = np.empty_like(psf)
+    np.divide(psf, s, out=out, dtype=np.float64, casting="same_kind")
+    return out
 
 
 def psf_autocrop(psf, imshape, s: DwOpts):
@@ -347,12 +350,15 @@ def psf_autocrop(psf, imshape, s: DwOpts):
 def xplane_sums_f32(psf):
     """Sum of each x plane of a (pP, pN, pM) PSF accumulated in float32 in
     deconwolf's order, y outer and z inner (psf_autocrop_XY, dw.c:1873-1882):
-    one sequential float32 accumulation per plane."""
-    a = np.ascontiguousarray(np.asarray(psf, dtype=np.float32).transpose(2, 1, 0))  # [x][y][z]
-    m = a.shape[0]
+    one sequential float32 accumulation per plane, all planes together (a sum
+    over the first axis of a C-ordered array adds row after row)."""
+    a = np.ascontiguousarray(np.asarray(psf, dtype=np.float32).transpose(1, 0, 2))  # [y][z][x]
+    m = a.shape[2]
     if a.size == 0:
         return np.zeros(m, np.float32)
-    return np.cumsum(a.reshape(m, -1), axis=1, dtype=np.float32)[:, -1].copy()
+    if m == 1:  # a single column would be summed pairwise
+        return np.cumsum(a.reshape(-1), dtype=np.float32)[-1:].copy()
+    return np.add.reduce(a.reshape(-1, m), axis=0, dtype=np.float32)
 
 
 def deconvolve(image, psf, iterations, bq=2, verbose=0, opts: Optional[DwOpts] = None):
@@ -365,7 +371,7 @@ def deconvolve(image, psf, iterations, bq=2, verbose=0, opts: Optional[DwOpts] =
     s.iter_type = ITER_FIXED
     s.borderQuality = int(bq)
     s.verbosity = int(verbose)
-    im = np.array(image, dtype=np.float32, copy=True)
+    im = np.asarray(image, dtype=np.float32)
     if im.min() < 0:
         raise ValueError("the image has negative values (dw.c:2703-2710)")
     if im.max() < 1:
@@ -374,7 +380,7 @@ def deconvolve(image, psf, iterations, bq=2, verbose=0, opts: Optional[DwOpts] =
     ps = psf_autocrop(ps, im.shape, s)
     ps = fim_normalize_sum1(ps)
     if s.offset > 0:
-        im += np.float32(s.offset)
+        im = im + np.float32(s.offset)  # the caller's array stays as it is
     if int(s.method) == METHOD_RL:
         return deconvolve_rl_hip(im, ps, s)
     return deconvolve_shb_hip(im, ps, s)

@@ -62,7 +62,18 @@ def to_u16(out, scaling, mode):
     dst = torch.empty(out.shape, dtype=torch.int16, device=out.device)
     check(lib().dwhip_to_u16_device(out.data_ptr(), out.numel(), float(scaling), int(mode), dst.data_ptr(),
                                     torch.cuda.current_stream().cuda_stream), "dwhip_to_u16_device")
-    return dst.cpu().numpy().view(np.uint16)
+    return to_host(dst).view(np.uint16)
+
+
+def to_host(t):
+    """A contiguous GPU tensor as a new numpy array."""
+    import torch
+    a = np.empty(tuple(t.shape), dtype={torch.int16: np.int16, torch.float32: np.float32}[t.dtype])
+    if a.nbytes:
+        with torch.cuda.device(t.device):
+            check(lib().dwhip_download(a.ctypes.data, t.data_ptr(), a.nbytes,
+                                       torch.cuda.current_stream().cuda_stream), "dwhip_download")
+    return a
 
 
 # ---------------------------------------------------------------------------
@@ -199,7 +210,7 @@ def imwrite(path, out, s, tiled=False, log=None):
             s.scaling = 1.0
             if log is not None:
                 log.write("scaling: %f\n" % s.scaling)
-        vol = out.contiguous().cpu().numpy()
+        vol = to_host(out.contiguous())
         write_npy(path, vol) if _is_npy(path) else write_tiff(path, vol)
         return None
     if tiled:

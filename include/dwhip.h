@@ -264,6 +264,13 @@ int dwhip_bw_psf_device(float *out, int64_t N, int64_t P, double lambda_nm, doub
                         double dxy_nm, double dz_nm, void *stream);
 
 /*
+ * Copies `bytes` from device memory to pageable host memory after what is
+ * queued on `stream`, and waits for it; several host threads share the copy
+ * of a large result (the page faults of new memory among it).
+ */
+int dwhip_download(void *dst, const void *src, size_t bytes, void *stream);
+
+/*
  * FFT check entry (device memory): unnormalised 3-D R2C of an nx*ny*nz
  * real volume (nx even) into (nx/2+1)*ny*nz complex, interleaved, the
  * layout of fftwf_plan_dft_r2c_3d(nz, ny, nx) that src/fft.c:236-290

@@ -126,3 +126,23 @@ def test_autocrop_factor_above_one_is_an_error():
     psf = gauss_psf(15, 7, 2.0, 3.0, rng)
     with pytest.raises(ValueError):
         ms.psf_autocrop(psf, (20, 64, 64), ms.DwOpts(xycropfactor=1.5))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (7, 5, 1), (1, 9, 2), (5, 1, 3), (33, 29, 31), (79, 181, 181)])
+@pytest.mark.parametrize("order", ["C", "F"])
+def test_xplane_sums_are_sequential(shape, order):
+    """The plane sums equal one float32 accumulation per plane, y outer and z
+    inner, bit for bit (values of very different size, so that any other
+    order rounds differently)."""
+    rng = np.random.default_rng(11)
+    psf = np.asarray(np.exp(rng.uniform(-12, 2, shape)).astype(np.float32), order=order)
+    ref = np.cumsum(psf.transpose(2, 1, 0).reshape(shape[2], -1), axis=1, dtype=np.float32)[:, -1]
+    np.testing.assert_array_equal(ms.xplane_sums_f32(psf), ref)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (5, 4, 3), (31, 33, 35)])
+def test_normalize_is_the_double_quotient(shape):
+    rng = np.random.default_rng(12)
+    psf = np.exp(rng.uniform(-12, 2, shape)).astype(np.float32)
+    ref = (psf.astype(np.float64) / float(np.sum(psf, dtype=np.float64))).astype(np.float32)
+    np.testing.assert_array_equal(ms.fim_normalize_sum1(psf), ref)

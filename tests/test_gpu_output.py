@@ -85,3 +85,37 @@ def test_imwrite_matches_reference_rules(tmp_path, name, tiled):
             got.append(np.array(im).astype(np.uint16))
         got = np.stack(got)
     assert got.dtype == np.uint16 and np.array_equal(got, want)
+
+
+# below and at the size from which several threads copy, one element more, a
+# last chunk of a few bytes, more chunks than threads
+@pytest.mark.parametrize("n", [1, (4 << 20) - 1, 4 << 20, (4 << 20) + 1, (9 << 20) + 3, (40 << 20) + 5])
+def test_to_host_is_the_tensor(n):
+    print("to_host", n, flush=True)
+    t = (torch.arange(n, device=DEV, dtype=torch.int32) * 7919 % 65521 - 32760).to(torch.int16)
+    a = output.to_host(t)
+    assert a.dtype == np.int16 and np.array_equal(a, t.cpu().numpy())
+    f = t[: n // 2 + 1].float()
+    assert np.array_equal(output.to_host(f), f.cpu().numpy())
+
+
+def test_to_host_from_threads_and_streams():
+    """Copies from several host threads, each on its own stream after work
+    queued there: one shares the staging buffers, the others copy plainly."""
+    import threading
+    got = [None] * 4
+
+    def one(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            t = torch.full((6 << 20,), float(i + 1), device=DEV)
+            t.mul_(3.0)
+            got[i] = output.to_host(t)
+
+    th = [threading.Thread(target=one, args=(i,)) for i in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for i in range(4):
+        assert np.all(got[i] == 3.0 * (i + 1))
