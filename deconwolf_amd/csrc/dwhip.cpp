@@ -327,7 +327,7 @@ static int pow2_floor(int v)
     return p;
 }
 
-// x tiles of pass E for SHB: ceil(N / xrows) tiles in each of the P planes
+// x tiles of a pruned pass E: ceil(N / xrows) tiles in each of the P planes
 static int ratio_tiles(int64_t N, int64_t P, int xrows)
 {
     return (int)(((N + xrows - 1) / xrows) * P);
@@ -543,6 +543,9 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     d.M = (int)M; d.N = (int)N; d.P = (int)P;
     d.pM = (int)pM; d.pN = (int)pN; d.pP = (int)pP;
     d.refMNP = (double)ref[0] * (double)ref[1] * (double)ref[2];
+    d.rl = prm->method == DWHIP_METHOD_RL;
+    d.has_w = prm->border_quality > 0;
+    d.prune = !d.rl || d.has_w || (M == w[0] && N == w[1] && P == w[2]);
     // plan: the autotuner's candidate, else a measured plan from the cache,
     // else the rule planner's
     DwhipPlanChoice cached;
@@ -560,14 +563,12 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
         t.ntile[KIND_Y] = t.ntile[KIND_Y] / d.nz * d.uz;
     }
     {
-        // pass D transforms slabs z < P; pass F too, except for RL, whose
-        // ratio is 1e-6 outside the image
+        // pass D transforms slabs z < P; pass F and pass E's rows y < N too
+        // when the job is pruned
         const int nct = (d.hc + j->tiles.ycols - 1) / j->tiles.ycols;
         j->tiles.ntile[KIND_YD] = nct * (int)P;
-        j->tiles.ntile[KIND_YF] = prm->method == DWHIP_METHOD_RL ? nct * d.uz : nct * (int)P;
-        // pass E: rows y < N of planes z < P for SHB (whose ratio is 0
-        // elsewhere), all rows for RL
-        if (prm->method != DWHIP_METHOD_RL) j->tiles.ntile[KIND_XR] = ratio_tiles(N, P, j->tiles.xrows);
+        j->tiles.ntile[KIND_YF] = nct * (d.prune ? (int)P : d.uz);
+        if (d.prune) j->tiles.ntile[KIND_XR] = ratio_tiles(N, P, j->tiles.xrows);
     }
     for (int k = 0; k < KIND_N; ++k) d.ntile[k] = j->tiles.ntile[k];
     d.xrows = j->tiles.xrows;
@@ -575,11 +576,9 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     d.zcols = j->tiles.zcols;
     d.positivity = prm->positivity;
     d.metric = prm->metric;
-    d.has_w = prm->border_quality > 0;
     d.bg_auto = prm->bg_auto;
     d.start_identity = prm->start != DWHIP_START_FLAT;
     d.niter = niter;
-    d.rl = prm->method == DWHIP_METHOD_RL;
     d.iter_type = prm->iter_type;
     d.err_rel = prm->err_rel;
     d.err_abs = prm->err_abs;
@@ -748,9 +747,9 @@ double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
     if (!xkind) {
         switch (mode) {
         case CM_ZCONV: return Vc + Kc + slabP;                 // read C, K; write z < P
-        case CM_ZCONVJ: return (d.rl ? Vc : slabP) + Kc + Vc;  // read z < P (RL: all), K; write C
+        case CM_ZCONVJ: return (d.prune ? slabP : Vc) + Kc + Vc;  // read z < P (or all), K; write C
         case CM_YINV_IMG: return slabP + imgrows;              // slabs z < P, write y < N
-        case CM_YFWD_IMG: return d.rl ? Xc + Vc : imgrows + slabP;
+        case CM_YFWD_IMG: return d.prune ? imgrows + slabP : Xc + Vc;
         case CM_YFWD:
         case CM_YINV: return Xc + Vc;
         default: return 2 * Vc;
@@ -765,7 +764,7 @@ double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
         // (and W), writes x_k
         if (iter == 0) return (d.rl ? 1 : 2) * V + Xc;
         return 2 * Xc + ((d.rl ? 2 : 3) + (d.has_w ? 1 : 0)) * V;
-    case XM_RATIO: return d.rl ? imgrows + Xc + img : 2 * imgrows + img;
+    case XM_RATIO: return d.prune ? 2 * imgrows + img : imgrows + Xc + img;
     case XM_LOAD: return Vc + V;
     case XM_STORE: return Vc + V;
     default: return 0;

@@ -12,9 +12,9 @@
 
 // Tile spaces: x-row tiles, y column tiles of all slabs, z column tiles,
 // and the tiles of the pruned passes — KIND_YD: slabs z < P (pass D);
-// KIND_YF: pass F's slabs (z < P for SHB, all of them for RL); KIND_XR:
-// pass E's rows (for SHB the rows y < N of the planes z < P, in tiles that
-// stay within one plane; for RL all x tiles).  A pruned pass enumerates only
+// KIND_YF: pass F's slabs (z < P, or all of them without pruning); KIND_XR:
+// pass E's rows (the rows y < N of the planes z < P, in tiles that stay
+// within one plane; all x tiles without pruning, see JobDev.prune).  A pruned pass enumerates only
 // the tiles it works on, so its grid carries no idle workgroups and every
 // XCD gets a share of the work.
 enum { KIND_X = 0, KIND_Y = 1, KIND_Z = 2, KIND_YD = 3, KIND_YF = 4, KIND_XR = 5, KIND_N = 6 };
@@ -65,6 +65,12 @@ struct JobDev {
     int start_identity; // start from start_img (or im) inserted, instead of flat
     int niter;          // iterations requested (nIter, or maxiter for REL/ABS)
     int rl;             // 1: Richardson-Lucy (method_rl.c), 0: SHB (method_shb.c)
+    // 1: the adjoint half runs on the image's rows and planes alone.  The SHB
+    // ratio is 0 outside the image; RL's is 1e-6 there, whose adjoint is known
+    // (1e-6 times the PSF's sum, less what the image box covers, P1 = 1/W of
+    // the Bertero weights) and added in the update.  0: RL without weights on
+    // a period that exceeds the image.
+    int prune;
     // stopping rule (dw_iterator_next, src/dw.c:237-269)
     int iter_type;      // DWHIP_DEV_ITER_*
     float err_rel, err_abs;

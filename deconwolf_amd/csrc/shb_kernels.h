@@ -8,8 +8,8 @@
 // LOAD (R2C of U0), STORE (C2R into U0, unnormalised).
 enum { XM_PSF = 0, XM_ONES = 1, XM_WEIGHTS = 2, XM_UPDATE = 3, XM_RATIO = 4, XM_LOAD = 5, XM_STORE = 6 };
 // Column-pass modes; ZOTF: forward, divide by nx*ny*nz, store into K.
-// Pruned modes of the SHB iteration (the skipped values are exact zeros or
-// never read): ZCONV writes only z < P; ZCONVJ reads only z < P; YINV_IMG
+// Pruned modes of the iteration (the skipped values are exact zeros or
+// never read, JobDev.prune): ZCONV writes only z < P; ZCONVJ reads only z < P; YINV_IMG
 // (pass D) transforms only slabs z < P and writes only y < N; YFWD_IMG
 // (pass F) reads only y < N of slabs z < P and skips the other slabs.
 enum { CM_YFWD = 0, CM_YINV = 1, CM_ZOTF = 2, CM_ZCONV = 3, CM_ZCONVJ = 4, CM_ZFWD = 5, CM_ZINV = 6,

@@ -50,6 +50,15 @@ __device__ __forceinline__ double shb_alpha(int iter, float alphamax)
     return a;
 }
 
+// Richardson-Lucy step x~ (f W) (method_rl.c:85-97) of a pruned job: x~ lacks
+// the adjoint of the ratio's 1e-6 outside the image, 1e-6 (S - P1) with S the
+// PSF's sum and P1 = 1/W; times f W that is 1e-6 f (S W - 1).  W = 0 (P1 below
+// method_rl.c's limit) gives 0 either way.
+__device__ __forceinline__ float rl_step(float xt, float f, float w, float psum)
+{
+    return w > 0.f ? fmaf(1e-6f * f, fmaf(psum, w, -1.f), xt * (f * w)) : 0.f;
+}
+
 // p = x + alpha*(x - xp), then p = max(p, bg)  (method_shb.c:333-339):
 // x - xp in float, the rest in double, rounded to float.  With
 // DWHIP_EXTRAP_F32 the product and sum are one float FMA with alpha rounded
@@ -283,14 +292,10 @@ __host__ __device__ constexpr bool x_nt(int mode) { return mode == XM_UPDATE ? D
 #define DWHIP_NT_STATE 1
 #endif
 
-// Element loops of the two iteration passes specialised for their common
-// case (SHB iteration k > 0 of the update pass; the SHB ratio pass, whose
-// tiles hold image rows only): contiguous tile addressing, the job's flags
-// read once, selects instead of branches.  0 runs the generic loop for
-// every case (a build tunable for measurement).
-#ifndef DWHIP_X_FAST
-#define DWHIP_X_FAST 1
-#endif
+// The two iteration passes have element loops of their own for iteration k > 0
+// of the update pass (SHB, RL) and for the pruned ratio pass, whose tiles hold
+// image rows only: contiguous tile addressing, the job's flags read once,
+// selects instead of branches.  Everything else runs the generic loop.
 
 #ifdef DWHIP_X_WAVES
 #define DWHIP_X_OCC __attribute__((amdgpu_waves_per_eu(DWHIP_X_WAVES)))
@@ -350,18 +355,17 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         int urow0 = row0;  // the tile's first row in the real volumes
         int ez = 0, ey0 = 0;
         if (EXT) {
-            const int rows = (MODE == XM_RATIO && !J.rl) ? J.N : J.uy;
+            const int rows = (MODE == XM_RATIO && J.prune) ? J.N : J.uy;
             const int tpp = (rows + J.xrows - 1) / J.xrows;
             ez = lt / tpp;
             ey0 = (lt - ez * tpp) * J.xrows;
             row0 = ez * ny + ey0;
             urow0 = ez * J.uy + ey0;
             nrows = min(J.xrows, rows - ey0);
-        } else if (MODE == XM_RATIO && !J.rl) {
-            // the SHB ratio is 0 outside the image box and only y < N, z < P
-            // rows of y are used: pass E's tiles cover exactly those rows,
-            // ceil(N / xrows) tiles within each plane z < P (the RL ratio is
-            // 1e-6 outside the image, so RL runs the plain x tiles)
+        } else if (MODE == XM_RATIO && J.prune) {
+            // only rows y < N, z < P of y are used and the adjoint reads only
+            // those of the ratio: pass E's tiles cover exactly those rows,
+            // ceil(N / xrows) tiles within each plane z < P
             const int tpp = (J.N + J.xrows - 1) / J.xrows;
             const int z = lt / tpp, k = lt - z * tpp;
             row0 = z * ny + k * J.xrows;
@@ -469,16 +473,19 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         // alpha of iterations k-1 and k (uniform)
         const double am1 = MODE == XM_UPDATE ? shb_alpha(iter - 1, J.alphamax) : 0.0;
         const double al = MODE == XM_UPDATE ? shb_alpha(iter, J.alphamax) : 0.0;
-        // the SHB ratio pass's tiles lie within one plane: its rows' y and z
+        // the PSF's sum: the OTF's first value without its scale
+        const float psum =
+            MODE == XM_UPDATE && J.rl && J.has_w ? ldg(gp(J.K)).x * (((float)J.nx * (float)J.ny) * (float)J.nz) : 0.f;
+        // the pruned ratio pass's tiles lie within one plane: its rows' y and z
         // come from the tile (no division per element)
-        const bool plane_tile = EXT || (MODE == XM_RATIO && !J.rl);
+        const bool plane_tile = EXT || (MODE == XM_RATIO && J.prune);
         const int tz = EXT ? ez : plane_tile ? row0 / ny : 0;
         const int ty0 = EXT ? ey0 : plane_tile ? row0 - tz * ny : 0;
         // chunks of XCHUNK elements per thread; full chunks carry no bounds
         // tests, so their loads and arithmetic schedule as straight-line code
         auto chunk = [&](int w0, auto full) {
             using FULL = decltype(full);
-            float2 a[XCHUNK], b[XCHUNK], c[XCHUNK], wv[XCHUNK];
+            float2 a[XCHUNK], b[XCHUNK], c[XCHUNK];
             size_t vi[XCHUNK];
             int yy[XCHUNK], zz[XCHUNK], m0[XCHUNK];
 #pragma unroll
@@ -496,7 +503,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                 }
                 m0[q] = 2 * n;
                 vi[q] = (size_t)row * ux + 2 * n;
-                a[q] = b[q] = c[q] = wv[q] = make_float2(0.f, 0.f);
+                a[q] = b[q] = c[q] = make_float2(0.f, 0.f);
             }
 #pragma unroll
             for (int q = 0; q < XCHUNK; ++q) {
@@ -505,7 +512,6 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                 if (MODE == XM_UPDATE) {
                     b[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Ukm1 + vi[q]));
                     if (!J.rl) c[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Uk + vi[q]));
-                    if (iter > 0 && J.has_w) wv[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(W + vi[q]));
                 } else if (MODE == XM_LOAD) {
                     a[q] = ldg(reinterpret_cast<const DWHIP_GL float2*>(U0 + vi[q]));
                 } else if (MODE == XM_RATIO) {
@@ -547,51 +553,15 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                     out.x = p1.x > sigma ? (float)(1.0 / p1.x) : 0.f;
                     out.y = p1.y > sigma ? (float)(1.0 / p1.y) : 0.f;
                     stg(reinterpret_cast<DWHIP_GL float2*>(W + vi[q]), out);
-                } else if (MODE == XM_UPDATE && J.rl) {
-                    // Richardson-Lucy (method_rl.c:85-97, 357-366): f = x_{k-1},
-                    // x_k = x~ * (f * W), clamped to bg when bg > 0
-                    const float2 f = b[q];
-                    float2 xk = f;  // iteration 0: the start guess
-                    if (iter > 0) {
-                        const float2 xt = a[q];
-                        if (J.has_w)
-                            xk = make_float2(xt.x * (f.x * wv[q].x), xt.y * (f.y * wv[q].y));
-                        else
-                            xk = make_float2(xt.x * f.x, xt.y * f.y);
-                        if (bg > 0) {
-                            xk.x = xk.x < bg ? bg : xk.x;
-                            xk.y = xk.y < bg ? bg : xk.y;
-                        }
-                        stgs<XNT>(reinterpret_cast<DWHIP_GL float2*>(Uk + vi[q]), xk);
-                    }
-                    out = xk;
                 } else if (MODE == XM_UPDATE) {
-                    const float2 xkm1 = b[q];
-                    float2 xk;
-                    if (iter == 0) {
-                        xk = c[q];  // U0 = x_0, U1 = x_{-1} = x_0 (start guess)
-                    } else {
-                        // finish iteration k-1 (method_shb.c:55-70, 357-376)
-                        const float2 xt = a[q];
-                        const float2 xkm2 = c[q];
-                        const float p0 = shb_extrap(xkm1.x, xkm2.x, am1, bg);
-                        const float p1 = shb_extrap(xkm1.y, xkm2.y, am1, bg);
-                        if (J.has_w)
-                            xk = make_float2(xt.x * (p0 * wv[q].x), xt.y * (p1 * wv[q].y));
-                        else
-                            xk = make_float2(xt.x * p0, xt.y * p1);
-                        if (J.positivity) {
-                            xk.x = xk.x < bg ? bg : xk.x;
-                            xk.y = xk.y < bg ? bg : xk.y;
-                        }
-                        stgs<XNT>(reinterpret_cast<DWHIP_GL float2*>(Uk + vi[q]), xk);
-                    }
-                    out = make_float2(shb_extrap(xk.x, xkm1.x, al, bg), shb_extrap(xk.y, xkm1.y, al, bg));
+                    // iteration 0 (the later ones have their own loops): x_0 is
+                    // the start guess, and for SHB U1 = x_{-1} = x_0 too
+                    out = J.rl ? b[q] : make_float2(shb_extrap(c[q].x, b[q].x, al, bg), shb_extrap(c[q].y, b[q].y, al, bg));
                 } else {  // XM_RATIO, method_shb.c:27-48 and getError dw.c:1436-1524
                     const float2 yv = a[q];
                     // outside the image: 0 for SHB (method_shb.c:44), 1e-6 for RL
-                    // (method_rl.c:62)
-                    const float outside = J.rl ? 1e-6f : 0.f;
+                    // (method_rl.c:62), whose part a pruned job adds in the update
+                    const float outside = J.rl && !J.prune ? 1e-6f : 0.f;
                     float r[2] = {outside, outside};
                     if (yy[q] < J.N && zz[q] < J.P) {
 #pragma unroll
@@ -632,7 +602,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         const bool rl = J.rl;
         const bool has_w = J.has_w;
         const float lo = J.positivity ? bg : -INFINITY;  // x_k < lo -> lo (method_shb.c:366-374)
-        if (DWHIP_X_FAST && MODE == XM_UPDATE && !rl && iter > 0) {
+        if (MODE == XM_UPDATE && !rl && iter > 0) {
             // SHB iteration k > 0.  The tile's x-rows row0 .. row0+nrows-1
             // are consecutive in every real volume (row stride 2 * dp), so
             // packed pair w of the tile is pair w from the tile's first voxel.
@@ -676,16 +646,49 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                 rows(BoolC<true>());
             else
                 rows(BoolC<false>());
-        } else if (DWHIP_X_FAST && MODE == XM_RATIO && !J.rl && dp > 1) {
-            // SHB ratio over a plane tile: every row is an image row (y < N,
+        } else if (MODE == XM_UPDATE && rl && iter > 0) {
+            // RL iteration k > 0 (method_rl.c:85-97, 357-366), addressed as
+            // above; half a chunk at a time, so that the kernel's registers
+            // stay those of the SHB loop (four loads in flight per volume)
+            const size_t tb = (size_t)urow0 * ux;
+            const DWHIP_GL float2* __restrict__ xm1 = reinterpret_cast<const DWHIP_GL float2*>(Ukm1 + tb);
+            DWHIP_GL float2* __restrict__ xo = reinterpret_cast<DWHIP_GL float2*>(Uk + tb);
+            const DWHIP_GL float2* __restrict__ wt = reinterpret_cast<const DWHIP_GL float2*>(W + tb);
+            const float rlo = bg > 0 ? bg : -INFINITY;
+            constexpr int RC = XCHUNK / 2;
+            for (int w0 = tid; w0 < nwork; w0 += RC * XTHR) {
+                float2 f[RC], wv[RC];
+#pragma unroll
+                for (int q = 0; q < RC; ++q) {
+                    const int w = min(w0 + q * XTHR, nwork - 1);
+                    f[q] = ldgs<DWHIP_NT_STATE>(xm1 + w);
+                    wv[q] = has_w ? ldgs<DWHIP_NT_STATE>(wt + w) : make_float2(1.f, 1.f);
+                }
+#pragma unroll
+                for (int q = 0; q < RC; ++q) {
+                    const int w = w0 + q * XTHR;
+                    if (w >= nwork) continue;
+                    const float2 xt = lds[lix(w)];
+                    float2 xk = has_w ? make_float2(rl_step(xt.x, f[q].x, wv[q].x, psum),
+                                                    rl_step(xt.y, f[q].y, wv[q].y, psum))
+                                      : make_float2(xt.x * f[q].x, xt.y * f[q].y);
+                    xk.x = xk.x < rlo ? rlo : xk.x;
+                    xk.y = xk.y < rlo ? rlo : xk.y;
+                    stgs<DWHIP_NT_STATE>(xo + w, xk);
+                    lds[lix(w)] = xk;
+                }
+            }
+        } else if (MODE == XM_RATIO && J.prune && dp > 1) {
+            // ratio over a plane tile: every row is an image row (y < N,
             // z < P); pair w holds columns 2n, 2n+1 of tile row w / h.  Image
             // loads are clamped into the tile's rows and dropped beyond
-            // column M (method_shb.c:27-48, getError dw.c:1436-1524).
+            // column M (method_shb.c:27-48, method_rl.c:45-65, getError
+            // dw.c:1436-1524).
             const int M = J.M;
             const DWHIP_GL float* __restrict__ imt = im + (size_t)M * (ty0 + (size_t)J.N * tz);
             const int ilast = nrows * M - 1;
-            auto rat = [&](int w0, auto full, auto idiv) {
-                constexpr bool FULL = decltype(full)::value, IDIV = decltype(idiv)::value;
+            auto rat = [&](int w0, auto full, auto idiv, auto isrl) {
+                constexpr bool FULL = decltype(full)::value, IDIV = decltype(idiv)::value, RL = decltype(isrl)::value;
                 float2 a[XCHUNK], gv[XCHUNK];
                 int m0[XCHUNK];
 #pragma unroll
@@ -720,21 +723,31 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
                             term = (yd - gd) * (yd - gd);
                         acc += valid ? term : 0.0;
                         float rv = qt;
-                        if (fabs(yd) < 1e-6) rv = g / (float)copysign(1e-6, yd);  // method_shb.c:41-42
+                        if (RL)
+                            rv = y > 0 ? qt : bg;  // method_rl.c:52-60
+                        else if (fabs(yd) < 1e-6)
+                            rv = g / (float)copysign(1e-6, yd);  // method_shb.c:41-42
                         r[e] = valid ? rv : 0.f;
                     }
                     lds[lix(w)] = make_float2(r[0], r[1]);
                 }
             };
-            auto rows = [&](auto idiv) {
+            auto rows = [&](auto idiv, auto isrl) {
                 int w0 = tid;
-                for (; w0 + (XCHUNK - 1) * XTHR < nwork; w0 += XCHUNK * XTHR) rat(w0, BoolC<true>(), idiv);
-                for (; w0 < nwork; w0 += XCHUNK * XTHR) rat(w0, BoolC<false>(), idiv);
+                for (; w0 + (XCHUNK - 1) * XTHR < nwork; w0 += XCHUNK * XTHR) rat(w0, BoolC<true>(), idiv, isrl);
+                for (; w0 < nwork; w0 += XCHUNK * XTHR) rat(w0, BoolC<false>(), idiv, isrl);
             };
-            if (J.metric == DWHIP_DEV_METRIC_IDIV)
-                rows(BoolC<true>());
-            else
-                rows(BoolC<false>());
+            const bool idiv = J.metric == DWHIP_DEV_METRIC_IDIV;
+            if (rl) {
+                if (idiv)
+                    rows(BoolC<true>(), BoolC<true>());
+                else
+                    rows(BoolC<false>(), BoolC<true>());
+            } else if (idiv) {
+                rows(BoolC<true>(), BoolC<false>());
+            } else {
+                rows(BoolC<false>(), BoolC<false>());
+            }
         } else {
             int w0 = tid;
             for (; w0 + (XCHUNK - 1) * XTHR < nwork; w0 += XCHUNK * XTHR) chunk(w0, BoolC<true>());
@@ -767,7 +780,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             __syncthreads();
             [[maybe_unused]] const int hp = h / 2 + 1;
             DWHIP_GL float2* __restrict__ dst = gp(J.C) + (size_t)row0 * hcs;
-            // (the SHB ratio pass's plane tiles hold image rows only, so
+            // (the pruned ratio pass's plane tiles hold image rows only, so
             // every row of a tile is written)
 #if DWHIP_MERGE_BY_BIN == 2
             // a thread writes bin m (0 <= m <= h) of every row of the tile,
@@ -1049,7 +1062,7 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         g.npshift = __ffs(B) - 1;  // B is a power of two
         // elements read (i < nin) and written (i < nout) along the pencil
         const int nd = EXT ? (ykind ? J.uy : J.uz) : g.n;  // data values along the pencil
-        const int nin = (MODE == CM_YFWD_IMG && !J.rl) ? J.N : (MODE == CM_ZCONVJ && !J.rl) ? J.P
+        const int nin = (MODE == CM_YFWD_IMG && J.prune) ? J.N : (MODE == CM_ZCONVJ && J.prune) ? J.P
                         : (MODE == CM_YINV || MODE == CM_YINV_IMG) ? g.n : nd;
         const int nout = (MODE == CM_YINV_IMG) ? J.N : (MODE == CM_ZCONV) ? J.P
                          : (MODE == CM_YINV || MODE == CM_ZCONVJ) ? nd : g.n;

@@ -11,6 +11,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 import deconwolf_amd as dw
+from deconwolf_amd import synth
 from oracle import pyoracle as po
 from test_gpu_shb import DEV, case, rel_l2
 
@@ -123,3 +124,24 @@ def test_rl_device_entry_and_engine_bit_identical(groups):
     assert st1["iterations"] == 7 and st2["iterations"] == 5
     assert np.array_equal(o1.cpu().numpy(), a)
     assert np.array_equal(o2.cpu().numpy(), shb)
+
+
+# the adjoint of the ratio's 1e-6 outside the image, added in the update: PSFs
+# that do not sum to 1, one so wide that most of the work volume is outside the
+# image, bq 1 on fast sizes, bq 0 with and without an outside
+@pytest.mark.parametrize("shape,psf_shape,bq,scale", [
+    ((12, 20, 24), (7, 9, 9), 2, 3.0), ((6, 11, 13), (11, 21, 25), 2, 0.25), ((16, 26, 27), (7, 9, 9), 1, 1.0),
+    ((16, 30, 32), (7, 9, 9), 0, 1.0), ((6, 30, 32), (16, 9, 9), 0, 1.0)])
+@pytest.mark.parametrize("metric", [dw.METRIC_IDIV, dw.METRIC_MSE])
+def test_outside_ratio(shape, psf_shape, bq, scale, metric):
+    print("rl outside:", shape, psf_shape, bq, scale, metric, flush=True)
+    rng = np.random.default_rng(5)
+    pP, pN, pM = psf_shape
+    k = (synth.gaussian_psf(pM, pN, pP, 1.7, 1.5, 1.4) * np.float32(scale)).astype(np.float32)
+    im = synth.noisy_image(synth.point_sources(shape, 20, rng=rng), 60.0, rng=rng) + np.float32(5.0)
+    s = dw.DwOpts(nIter=6, iter_type=dw.ITER_FIXED, borderQuality=bq, method=dw.METHOD_RL, metric=metric)
+    out = dw.deconvolve_rl_hip(im, k, s)
+    o32, e32, _, _ = po.rl(im, k, niter=6, border_quality=bq, metric=metric, work=s.stats["work"])
+    err = float(np.linalg.norm(out.astype(np.float64) - o32) / np.linalg.norm(o32))
+    assert err <= 1e-5, err
+    np.testing.assert_allclose(s.err_trace, e32, rtol=1e-4)
