@@ -152,7 +152,7 @@ SIGNATURES = [
                                  ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double)]),
 ]
 
-N_PROFILE_KERNELS = 16
+N_PROFILE_KERNELS = 17
 
 
 def profile_enable(on=True):

@@ -22,7 +22,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libdwhip.so")
 
 N_XMODES = 7
-N_CMODES = 9
+N_CMODES = 10
 # modes compiled for extended jobs too (xmode_has_ext, cmode_has_ext)
 EXT_XMODES = (1, 2, 3, 4)
 EXT_CMODES = (0, 1, 3, 4, 7, 8)

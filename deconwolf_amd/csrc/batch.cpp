@@ -311,11 +311,12 @@ int setup(dwhip_engine* E, const std::vector<EngJob*>& fresh)
     if (fast.empty()) return DWHIP_OK;
     RCHK(table_build(&E->tsetup, fast, s));
     for (int i = 0; i < (int)fast.size(); ++i) {
-        ECHK(dwhip_launch_stats(E->tsetup.jd(), i, DWHIP_STAT_BLOCKS, s));
+        const JobDev& d = fast[i]->j.d;
+        ECHK(dwhip_launch_stats(E->tsetup.jd(), i, (int64_t)d.M * d.N * d.P, s));
         ECHK(dwhip_launch_start(E->tsetup.jd(), i, 1024, s));
     }
     RCHK(table_pass(E->tsetup, true, XM_PSF, s));
-    RCHK(table_pass(E->tsetup, false, CM_YFWD, s));
+    RCHK(table_pass(E->tsetup, false, CM_YFWD_PSF, s));
     RCHK(table_pass(E->tsetup, false, CM_ZOTF, s));
     std::vector<EngJob*> wj;
     for (EngJob* j : fast)
@@ -323,7 +324,7 @@ int setup(dwhip_engine* E, const std::vector<EngJob*>& fresh)
     if (!wj.empty()) {
         RCHK(table_build(&E->tweights, wj, s));
         RCHK(table_pass(E->tweights, true, XM_ONES, s));
-        RCHK(table_pass(E->tweights, false, CM_YFWD, s));
+        RCHK(table_pass(E->tweights, false, CM_YFWD_IMG, s));
         RCHK(table_pass(E->tweights, false, CM_ZCONVJ, s));
         RCHK(table_pass(E->tweights, false, CM_YINV, s));
         RCHK(table_pass(E->tweights, true, XM_WEIGHTS, s));
@@ -645,7 +646,7 @@ int dwhip_engine_step(dwhip_engine* E, int64_t* done_tags, int max_done, int* n_
         std::vector<EngJob*> run;
         for (EngJob* j : E->active) {
             if (j->nrun == 0 && j->prm.iter_type != DWHIP_ITER_FIXED && !keep_going(j, 0)) {
-                ECHK(dwhip_launch_crop(j->j.jd, 0, dwhip_result_iterate(j->j.d.rl != 0, 0), j->out, 1024, s));
+                ECHK(dwhip_launch_crop(j->j.jd, 0, dwhip_result_iterate(j->j.d.rl != 0, 0), j->out, (int64_t)j->j.d.N * j->j.d.P, s));
                 finished.push_back(j);
             } else {
                 run.push_back(j);
@@ -719,7 +720,7 @@ int dwhip_engine_step(dwhip_engine* E, int64_t* done_tags, int max_done, int* n_
         if (fin) {
             // SHB returns x_{n-1}; RL returns x_n, after one more update pass
             if (j->j.d.rl) RCHK(dwhip_job_final_update(&j->j, j->j.bd, j->j.jd, js[j]));
-            ECHK(dwhip_launch_crop(j->j.jd, 0, dwhip_result_iterate(j->j.d.rl != 0, j->nrun), j->out, 1024, js[j]));
+            ECHK(dwhip_launch_crop(j->j.jd, 0, dwhip_result_iterate(j->j.d.rl != 0, j->nrun), j->out, (int64_t)j->j.d.N * j->j.d.P, js[j]));
             finished.push_back(j);
         } else {
             still.push_back(j);

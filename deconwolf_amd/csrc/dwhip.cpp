@@ -381,7 +381,7 @@ size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int
         size_t b = hcs * L[1] * (work[2] + L[2]) * sizeof(float2) + (border_quality > 0 ? 3 : 2) * V * sizeof(float);
         b += (size_t)ratio_tiles(work[1], work[2], t.xrows) * sizeof(double);
         b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-        b += DWHIP_STAT_BLOCKS * 4 * sizeof(double) + 4096 + 2 * sizeof(JobDev);
+        b += 4096 + 2 * sizeof(JobDev);
         for (int d = 0; d < 3; ++d) b += 3 * (size_t)L[d] * sizeof(float2);
         return b;
     }
@@ -392,7 +392,7 @@ size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int
         size_t b = 2 * Vh * sizeof(float2) + (border_quality > 0 ? 3 : 2) * V * sizeof(float);
         b += (size_t)dwhip_generic_ratio_grid() * sizeof(double);
         b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-        b += DWHIP_STAT_BLOCKS * 4 * sizeof(double) + 4096 + sizeof(GenDev) + sizeof(JobDev);
+        b += 4096 + sizeof(GenDev) + sizeof(JobDev);
         for (int d = 0; d < 3; ++d) b += 8 * (size_t)work[d] * sizeof(float2);  // twiddles, chirps, filters
         return b;
     }
@@ -405,7 +405,7 @@ size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int
     b += (border_quality > 0 ? 3 : 2) * V * sizeof(float); // U0, U1, W
     b += (size_t)std::max(t.ntile[KIND_X], ratio_tiles(N, P, t.xrows)) * sizeof(double);
     b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-    b += DWHIP_STAT_BLOCKS * 4 * sizeof(double) + 4096;
+    b += 4096;
     (void)M;
     return b;
 }
@@ -609,7 +609,6 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
         lay.U1 = take(V * sizeof(float));
         lay.W = d.has_w ? take(V * sizeof(float)) : 0;
         lay.part = take((size_t)d.ntile[KIND_XR] * sizeof(double));
-        lay.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
         lay.err = take((size_t)niter * sizeof(float));
         lay.errd = take((size_t)niter * sizeof(double));
         lay.tw = take(j->tw.size() * sizeof(float2));
@@ -642,7 +641,6 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     lay.U1 = take(V * sizeof(float));
     lay.W = d.has_w ? take(V * sizeof(float)) : 0;
     lay.part = take((size_t)std::max(d.ntile[KIND_X], d.ntile[KIND_XR]) * sizeof(double));
-    lay.stat = take(DWHIP_STAT_BLOCKS * 4 * sizeof(double));
     lay.err = take((size_t)niter * sizeof(float));
     lay.errd = take((size_t)niter * sizeof(double));
     lay.tw = take(tw.size() * sizeof(float2));
@@ -668,7 +666,9 @@ int dwhip_job_bind(DwhipJob* j, void* mem, hipStream_t s)
     d.U1 = (float*)(base + L.U1);
     d.W = d.has_w ? (float*)(base + L.W) : nullptr;
     d.part = (double*)(base + L.part);
-    d.stat = (double*)(base + L.stat);
+    // the statistics' partials (32 bytes per 2048 image values) are read before
+    // the first transform writes C
+    d.stat = (double*)d.C;
     d.err = (float*)(base + L.err);
     d.errd = (double*)(base + L.errd);
     d.tw = (const float2*)(base + L.tw);
@@ -752,12 +752,14 @@ double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
         case CM_YFWD_IMG: return d.prune ? imgrows + slabP : Xc + Vc;
         case CM_YFWD:
         case CM_YINV: return Xc + Vc;
+        case CM_YFWD_PSF: return row * d.pP * ((double)d.pN + d.ny);
+        case CM_ZOTF: return row * d.ny * ((double)d.pP + d.nz);
         default: return 2 * Vc;
         }
     }
     switch (mode) {
-    case XM_PSF: return Kc + (double)d.pM * d.pN * d.pP * sizeof(float);
-    case XM_ONES: return Xc;
+    case XM_PSF: return row * d.pN * d.pP + (double)d.pM * d.pN * d.pP * sizeof(float);
+    case XM_ONES: return imgrows;
     case XM_WEIGHTS: return Xc + V;
     case XM_UPDATE:
         // SHB reads x_{k-1}, x_{k-2} (and W), writes x_k; RL reads x_{k-1}
@@ -807,25 +809,21 @@ int dwhip_job_setup(const DwhipJob* j, hipStream_t s)
 {
     if (j->generic) return dwhip_generic_setup(j, s);
     const DwhipTiles& t = j->tiles;
-    const int nblk = DWHIP_STAT_BLOCKS;
-    HIPCHK(dwhip_launch_stats(j->jd, 0, nblk, s));
+    HIPCHK(dwhip_launch_stats(j->jd, 0, (int64_t)j->d.M * j->d.N * j->d.P, s));
     HIPCHK(dwhip_launch_start(j->jd, 0, 1024, s));
     // OTF: shifted PSF -> R2C -> K / (nx*ny*nz)
     {
         const BatchDev* bd = j->ext ? j->obd : j->bd;
         const JobDev* jd = j->ext ? j->ojd : j->jd;
         RCHK(dwhip_pass_x(XM_PSF, j, bd, jd, j->ext ? j->otf_tiles[0] : t.ntile[KIND_X], t.lds[KIND_X], s));
-        RCHK(dwhip_pass_c(CM_YFWD, j, bd, jd, j->ext ? j->otf_tiles[1] : t.ntile[KIND_Y], t.lds[KIND_Y], s));
+        RCHK(dwhip_pass_c(CM_YFWD_PSF, j, bd, jd, j->ext ? j->otf_tiles[1] : t.ntile[KIND_Y], t.lds[KIND_Y], s));
         RCHK(dwhip_pass_c(CM_ZOTF, j, bd, jd, j->ext ? j->otf_tiles[2] : t.ntile[KIND_Z], t.lds[KIND_Z], s));
     }
     if (j->d.has_w) {
         // P1 = IFFT(conj(K) FFT(1_box)); W = P1 > 0.01 ? 1/P1 : 0
-        RCHK(dwhip_pass_x(XM_ONES, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
-        // (an extended job continues the box as the adjoint reads it)
-        if (j->ext)
-            RCHK(dwhip_pass_c(CM_YFWD_IMG, j, j->bd, j->jd, t.ntile[KIND_YF], t.lds[KIND_YF], s));
-        else
-            RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
+        // (weights imply pruning: the adjoint reads the image's rows alone)
+        RCHK(dwhip_pass_x(XM_ONES, j, j->bd, j->jd, t.ntile[KIND_XR], t.lds[KIND_XR], s));
+        RCHK(dwhip_pass_c(CM_YFWD_IMG, j, j->bd, j->jd, t.ntile[KIND_YF], t.lds[KIND_YF], s));
         RCHK(dwhip_pass_c(CM_ZCONVJ, j, j->bd, j->jd, t.ntile[KIND_Z], t.lds[KIND_Z], s));
         RCHK(dwhip_pass_c(CM_YINV, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
         RCHK(dwhip_pass_x(XM_WEIGHTS, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
@@ -970,7 +968,7 @@ static int hooked_loop(DwhipJob* job, const dwhip_params* prm, float* out, hipSt
         const float* xh = nullptr;
         if (prm->hook_every > 0 && k % prm->hook_every == 0) {
             // x_k: RL's rounds end with x_k in U[k & 1] as SHB's do
-            HIPCHK(dwhip_launch_crop(job->jd, 0, k, out, 1024, s));
+            HIPCHK(dwhip_launch_crop(job->jd, 0, k, out, (int64_t)d.N * d.P, s));
             HIPCHK(hipMemcpyAsync(hx.data(), out, n_img * sizeof(float), hipMemcpyDeviceToHost, s));
             xh = hx.data();
         }
@@ -1082,7 +1080,7 @@ static int run_job(const float* im, int64_t M, int64_t N, int64_t P, const float
         // with no iteration run (REL stopping before iteration 0) the result
         // is the start guess x_0, which the swap-back of method_shb.c:385-390
         // hands back (deconvolve_rl would crop a NULL iterate there)
-        hipError_t e = dwhip_launch_crop(job.jd, 0, dwhip_result_iterate(job.d.rl != 0, nrun), out, 1024, s);
+        hipError_t e = dwhip_launch_crop(job.jd, 0, dwhip_result_iterate(job.d.rl != 0, nrun), out, N * P, s);
         if (e != hipSuccess) rc = dwhip_hip_fail(e, "crop", __LINE__);
     }
     hipError_t e = hipStreamSynchronize(s);

@@ -10,8 +10,7 @@
 #include "dwhip.h"
 #include "generic_dev.h"
 #include "shb_dev.h"
-
-#define DWHIP_STAT_BLOCKS 256
+#include "shb_kernels.h"
 
 struct DwhipTiles {
     int xrows, ycols, zcols;
@@ -29,7 +28,7 @@ struct DwhipPlanChoice {
 
 // Byte offsets of a job's buffers inside its device block.
 struct DwhipLayout {
-    size_t C, K, U0, U1, W, part, stat, err, errd, tw, st, tab, otab;
+    size_t C, K, U0, U1, W, part, err, errd, tw, st, tab, otab;
 };
 
 // One job: host copy of its descriptor plus its device block, which also
@@ -78,8 +77,8 @@ inline int dwhip_result_iterate(bool rl, int nrun)
 }
 
 // profiling of pass launches (profile.cpp); kernel ids: X modes 0..6, then
-// column modes 7..15
-#define DWHIP_PROF_KERNELS 16
+// column modes 7..16
+#define DWHIP_PROF_KERNELS 17
 bool dwhip_prof_on();
 int dwhip_prof_begin(hipStream_t s);
 void dwhip_prof_end(hipStream_t s, int slot, int kernel, double bytes);

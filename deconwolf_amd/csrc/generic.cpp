@@ -22,9 +22,6 @@ hipError_t dwhip_gen_launch_axis(const GenDev* gd, int axis, int sign, int grid,
                                  hipStream_t s);
 hipError_t dwhip_gen_launch_elem(const GenDev* gd, int op, int grid, hipStream_t s);
 hipError_t dwhip_gen_lds_limit(size_t bytes);
-hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int nblk, hipStream_t s);
-hipError_t dwhip_launch_start(const JobDev* jobs, int j, int grid, hipStream_t s);
-hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int njobs, int advance, hipStream_t s);
 }
 
 namespace {
@@ -290,7 +287,7 @@ int convolve(const DwhipJob* j, bool conj, hipStream_t s)
 // OTF, Bertero weights and start guess (method_shb.c:108-294).
 int dwhip_generic_setup(const DwhipJob* j, hipStream_t s)
 {
-    hipError_t e = dwhip_launch_stats(j->jd, 0, DWHIP_STAT_BLOCKS, s);
+    hipError_t e = dwhip_launch_stats(j->jd, 0, (int64_t)j->d.M * j->d.N * j->d.P, s);
     if (e == hipSuccess) e = dwhip_launch_start(j->jd, 0, 1024, s);
     if (e != hipSuccess) return dwhip_hip_fail(e, "any-size set-up", __LINE__);
     GCHK(elem(j, OP_PSF, s));

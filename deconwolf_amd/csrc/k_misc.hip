@@ -28,6 +28,26 @@ __device__ __forceinline__ double block_sum(double v, double* red)
 // Setup statistics: min(im) and sum(im) (bg_auto, flat start) and argmax(psf)
 // ---------------------------------------------------------------------------
 #define STHR 256
+// (min, sum, max, index of the max) of the workgroup's threads into element 0
+__device__ __forceinline__ void stats_reduce(int tid, double* smin, double* ssum, double* smax, double* sidx,
+                                             double vmin, double vsum, double vmax, double vidx)
+{
+    smin[tid] = vmin; ssum[tid] = vsum; smax[tid] = vmax; sidx[tid] = vidx;
+    __syncthreads();
+    for (int s = STHR / 2; s > 0; s >>= 1) {
+        if (tid < s) {
+            smin[tid] = fmin(smin[tid], smin[tid + s]);
+            ssum[tid] += ssum[tid + s];
+            const double m2 = smax[tid + s], i2 = sidx[tid + s];
+            if (m2 > smax[tid] || (m2 == smax[tid] && i2 < sidx[tid])) {
+                smax[tid] = m2;
+                sidx[tid] = i2;
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // stat layout per job: [nblk][4] doubles: min, sum, max, argmax index
 __global__ __launch_bounds__(STHR) void k_stats_partial(const JobDev* __restrict__ jobs, int j, int nblk)
 {
@@ -64,32 +84,22 @@ __global__ __launch_bounds__(STHR) void k_stats_partial(const JobDev* __restrict
         }
     }
     const int tid = threadIdx.x;
-    smin[tid] = vmin; ssum[tid] = vsum; smax[tid] = vmax; sidx[tid] = vidx;
-    __syncthreads();
-    for (int s = STHR / 2; s > 0; s >>= 1) {
-        if (tid < s) {
-            smin[tid] = fmin(smin[tid], smin[tid + s]);
-            ssum[tid] += ssum[tid + s];
-            const double m2 = smax[tid + s], i2 = sidx[tid + s];
-            if (m2 > smax[tid] || (m2 == smax[tid] && i2 < sidx[tid])) {
-                smax[tid] = m2;
-                sidx[tid] = i2;
-            }
-        }
-        __syncthreads();
-    }
+    stats_reduce(tid, smin, ssum, smax, sidx, vmin, vsum, vmax, vidx);
     if (tid == 0) {
         double* o = J.stat + 4 * (size_t)blockIdx.x;
         o[0] = smin[0]; o[1] = ssum[0]; o[2] = smax[0]; o[3] = sidx[0];
     }
 }
 
+// One workgroup adds the partials up (one thread walking 256 of them took
+// 45 us, a tenth of a small job).
 __global__ __launch_bounds__(STHR) void k_stats_final(const JobDev* __restrict__ jobs, int j, int nblk)
 {
     const JobDev& J = jobs[j];
-    if (threadIdx.x != 0) return;
+    __shared__ double smin[STHR], ssum[STHR], smax[STHR], sidx[STHR];
     double vmin = INFINITY, vsum = 0, vmax = -INFINITY, vidx = 1e300;
-    for (int b = 0; b < nblk; ++b) {
+    const int tid = threadIdx.x;
+    for (int b = tid; b < nblk; b += STHR) {
         const double* o = J.stat + 4 * (size_t)b;
         vmin = fmin(vmin, o[0]);
         vsum += o[1];
@@ -98,6 +108,11 @@ __global__ __launch_bounds__(STHR) void k_stats_final(const JobDev* __restrict__
             vidx = o[3];
         }
     }
+    stats_reduce(tid, smin, ssum, smax, sidx, vmin, vsum, vmax, vidx);
+    if (tid != 0) return;
+    vmin = smin[0];
+    vsum = ssum[0];
+    vidx = sidx[0];
     JobState* st = J.st;
     // bg_auto: bg = max(min(im), 1e-2)  (method_shb.c:108-117)
     float bg = J.bg_user;
@@ -231,6 +246,7 @@ DECL_LAUNCH(dwhip_launch_c5)
 DECL_LAUNCH(dwhip_launch_c6)
 DECL_LAUNCH(dwhip_launch_c7)
 DECL_LAUNCH(dwhip_launch_c8)
+DECL_LAUNCH(dwhip_launch_c9)
 DECL_LAUNCH(dwhip_launch_ce0)
 DECL_LAUNCH(dwhip_launch_ce1)
 DECL_LAUNCH(dwhip_launch_ce3)
@@ -257,18 +273,22 @@ hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDe
 hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
                                 hipStream_t s)
 {
-    static_assert(CM_YFWD == 0 && CM_YFWD_IMG == 8 && DWHIP_N_CMODES == 9, "column modes 0..8");
+    static_assert(CM_YFWD == 0 && CM_YFWD_PSF == 9 && DWHIP_N_CMODES == 10, "column modes 0..9");
     static const pass_launch f[2][DWHIP_N_CMODES] = {
         {dwhip_launch_c0, dwhip_launch_c1, dwhip_launch_c2, dwhip_launch_c3, dwhip_launch_c4, dwhip_launch_c5,
-         dwhip_launch_c6, dwhip_launch_c7, dwhip_launch_c8},
+         dwhip_launch_c6, dwhip_launch_c7, dwhip_launch_c8, dwhip_launch_c9},
         {dwhip_launch_ce0, dwhip_launch_ce1, nullptr, dwhip_launch_ce3, dwhip_launch_ce4, nullptr, nullptr,
-         dwhip_launch_ce7, dwhip_launch_ce8}};
+         dwhip_launch_ce7, dwhip_launch_ce8, nullptr}};
     if (mode < 0 || mode >= DWHIP_N_CMODES || !f[ext ? 1 : 0][mode]) return hipErrorInvalidValue;
     return f[ext ? 1 : 0][mode](bd, jobs, grid, lds, s);
 }
 
-hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int nblk, hipStream_t s)
+hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s)
 {
+    // at least eight values per thread (their loads are issued together), and
+    // four workgroups per CU for a large image: 1024 x 1024 x 60 takes
+    // 63 us (113 with one per CU)
+    const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(DWHIP_STAT_BLOCKS, nvox / (8 * STHR)));
     hipLaunchKernelGGL(k_stats_partial, dim3(nblk), dim3(STHR), 0, s, jobs, j, nblk);
     hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(STHR), 0, s, jobs, j, nblk);
     return hipGetLastError();
@@ -286,8 +306,11 @@ hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int nj
     return hipGetLastError();
 }
 
-hipError_t dwhip_launch_crop(const JobDev* jobs, int j, int k, float* out, int grid, hipStream_t s)
+hipError_t dwhip_launch_crop(const JobDev* jobs, int j, int k, float* out, int64_t nrows, hipStream_t s)
 {
+    // one row per workgroup as far as that goes: 1024 x 1024 x 60 in
+    // 110 us (158 with 1024 workgroups)
+    const int grid = (int)std::min<int64_t>(nrows, 1 << 16);
     hipLaunchKernelGGL(k_crop, dim3(grid), dim3(STHR), 0, s, jobs, j, k, out);
     return hipGetLastError();
 }

@@ -7,17 +7,17 @@
 // WEIGHTS (C2R, Bertero weights), UPDATE (pass A), RATIO (pass E),
 // LOAD (R2C of U0), STORE (C2R into U0, unnormalised).
 enum { XM_PSF = 0, XM_ONES = 1, XM_WEIGHTS = 2, XM_UPDATE = 3, XM_RATIO = 4, XM_LOAD = 5, XM_STORE = 6 };
-// Column-pass modes; ZOTF: forward, divide by nx*ny*nz, store into K.
+// Column-pass modes; YFWD_PSF and ZOTF: the PSF's transform, reading only the
+// rows and planes it covers (ZOTF: forward, divide by nx*ny*nz, store into K).
 // Pruned modes of the iteration (the skipped values are exact zeros or
 // never read, JobDev.prune): ZCONV writes only z < P; ZCONVJ reads only z < P; YINV_IMG
 // (pass D) transforms only slabs z < P and writes only y < N; YFWD_IMG
 // (pass F) reads only y < N of slabs z < P and skips the other slabs.
 enum { CM_YFWD = 0, CM_YINV = 1, CM_ZOTF = 2, CM_ZCONV = 3, CM_ZCONVJ = 4, CM_ZFWD = 5, CM_ZINV = 6,
-       CM_YINV_IMG = 7, CM_YFWD_IMG = 8 };
-#define DWHIP_N_CMODES 9
+       CM_YINV_IMG = 7, CM_YFWD_IMG = 8, CM_YFWD_PSF = 9 };
+#define DWHIP_N_CMODES 10
 // Passes an extended job runs (JobDev.ext): its OTF is set up by the plain
-// passes at the transform size, and its weights by YFWD_IMG (the ones box is
-// zero where that pass does not read).
+// passes at the transform size.
 __host__ __device__ constexpr bool xmode_has_ext(int m)
 {
     return m == XM_ONES || m == XM_WEIGHTS || m == XM_UPDATE || m == XM_RATIO;
@@ -28,10 +28,11 @@ __host__ __device__ constexpr bool cmode_has_ext(int m)
 }
 __host__ __device__ constexpr bool cmode_is_y(int m)
 {
-    return m == CM_YFWD || m == CM_YINV || m == CM_YINV_IMG || m == CM_YFWD_IMG;
+    return m == CM_YFWD || m == CM_YINV || m == CM_YINV_IMG || m == CM_YFWD_IMG || m == CM_YFWD_PSF;
 }
 // tile space of an x mode
-__host__ __device__ constexpr int xmode_kind(int m) { return m == XM_RATIO ? KIND_XR : KIND_X; }
+__host__ __device__ constexpr bool xmode_image_rows(int m) { return m == XM_RATIO || m == XM_ONES; }
+__host__ __device__ constexpr int xmode_kind(int m) { return xmode_image_rows(m) ? KIND_XR : KIND_X; }
 // tile space of a column mode
 __host__ __device__ constexpr int cmode_kind(int m)
 {
@@ -66,6 +67,7 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #define DWHIP_XROWS_MAX 64  // rows per X tile at most
 #endif
 #define DWHIP_MAX_RADIX 25
+#define DWHIP_STAT_BLOCKS 1024  // workgroups of the set-up statistics at most
 #ifndef DWHIP_X_STAGE_LDS
 #define DWHIP_X_STAGE_LDS 1  // X passes stage their half-spectrum rows in LDS before the C2R
 #endif
@@ -74,10 +76,10 @@ extern "C" {
 // ext: 1 launches the kernels of extended jobs (a table holds one kind)
 hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
 hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
-hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int nblk, hipStream_t s);
+hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s);
 hipError_t dwhip_launch_start(const JobDev* jobs, int j, int grid, hipStream_t s);
 hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int njobs, int advance, hipStream_t s);
-hipError_t dwhip_launch_crop(const JobDev* jobs, int j, int k, float* out, int grid, hipStream_t s);
+hipError_t dwhip_launch_crop(const JobDev* jobs, int j, int k, float* out, int64_t nrows, hipStream_t s);
 hipError_t dwhip_launch_tile_extract(const float* im, int M, int N, int x0, int y0, int z0, int xm, int xn, int xp,
                                      float offset, float* out, hipStream_t s);
 hipError_t dwhip_launch_tile_blend(const TileDev* tiles, int ntiles, int M, int N, int P, float offset, float* out,

@@ -77,6 +77,10 @@ __device__ __forceinline__ float shb_extrap(float x, float xp, double alpha, flo
     return p < bg ? bg : p;
 }
 
+// Whether value i of an axis of n values holds the PSF, p values moved so that
+// its value mid is at the origin.
+__device__ __forceinline__ bool psf_covers(int i, int mid, int n, int p) { return (i + mid) % n < p; }
+
 // Extended jobs: a convolution of period n with a PSF of p values, its
 // maximum at mid, as one of length L >= n + p - 1.  Output i < n of the
 // forward model reads inputs i - (p - 1 - mid) .. i + mid, the adjoint's
@@ -355,16 +359,17 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         int urow0 = row0;  // the tile's first row in the real volumes
         int ez = 0, ey0 = 0;
         if (EXT) {
-            const int rows = (MODE == XM_RATIO && J.prune) ? J.N : J.uy;
+            const int rows = (xmode_image_rows(MODE) && J.prune) ? J.N : J.uy;
             const int tpp = (rows + J.xrows - 1) / J.xrows;
             ez = lt / tpp;
             ey0 = (lt - ez * tpp) * J.xrows;
             row0 = ez * ny + ey0;
             urow0 = ez * J.uy + ey0;
             nrows = min(J.xrows, rows - ey0);
-        } else if (MODE == XM_RATIO && J.prune) {
+        } else if (xmode_image_rows(MODE) && J.prune) {
             // only rows y < N, z < P of y are used and the adjoint reads only
-            // those of the ratio: pass E's tiles cover exactly those rows,
+            // those of the ratio (and of the weights' ones): tiles cover
+            // exactly those rows,
             // ceil(N / xrows) tiles within each plane z < P
             const int tpp = (J.N + J.xrows - 1) / J.xrows;
             const int z = lt / tpp, k = lt - z * tpp;
@@ -372,6 +377,17 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             nrows = min(J.xrows, J.N - k * J.xrows);
         }
         const DWHIP_GL JobState* __restrict__ st = gp(J.st);
+        if (MODE == XM_PSF) {
+            // tiles without a row of the PSF stay unwritten (YFWD_PSF and ZOTF
+            // read the rows and planes it covers): 378 -> 129 us for 181 x 181 x
+            // 79 at 1250 x 1215 x 140, the two column passes 770 -> 637
+            bool any = false;
+            for (int b = 0; b < nrows; ++b) {
+                const int z = (row0 + b) / ny, y = (row0 + b) - z * ny;
+                any |= psf_covers(y, st->mid[1], ny, J.pN) && psf_covers(z, st->mid[2], J.nz, J.pP);
+            }
+            if (!any) return;
+        }
         const int iter = (MODE == XM_UPDATE || MODE == XM_RATIO) ? st->iter : 0;
         const bool inv = MODE == XM_RATIO || MODE == XM_WEIGHTS || MODE == XM_STORE ||
                          (MODE == XM_UPDATE && iter > 0);
@@ -478,7 +494,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             MODE == XM_UPDATE && J.rl && J.has_w ? ldg(gp(J.K)).x * (((float)J.nx * (float)J.ny) * (float)J.nz) : 0.f;
         // the pruned ratio pass's tiles lie within one plane: its rows' y and z
         // come from the tile (no division per element)
-        const bool plane_tile = EXT || (MODE == XM_RATIO && J.prune);
+        const bool plane_tile = EXT || (xmode_image_rows(MODE) && J.prune);
         const int tz = EXT ? ez : plane_tile ? row0 / ny : 0;
         const int ty0 = EXT ? ey0 : plane_tile ? row0 - tz * ny : 0;
         // chunks of XCHUNK elements per thread; full chunks carry no bounds
@@ -992,6 +1008,26 @@ struct WrapPencils {
     }
 };
 
+// Input pencils of the PSF's transform: zero where the PSF does not reach.
+template <bool NT>
+struct PsfPencils {
+    const DWHIP_GL float2* p;
+    size_t stride;
+    int npv;
+    int n, mid, len;
+    static constexpr bool kStrided = true;
+    __device__ __forceinline__ float2 operator()(int pen, int i) const
+    {
+        return (pen < npv && psf_covers(i, mid, n, len)) ? ldgs<NT>(p + i * stride + pen) : make_float2(0.f, 0.f);
+    }
+    template <int R>
+    __device__ __forceinline__ void load(int pen, int j, int nb, float2* v) const
+    {
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = (*this)(pen, j + r * nb);
+    }
+};
+
 // Workgroup b runs on XCD b mod 8 (dispatch is round robin over the 8 XCDs,
 // each with its own L2).  Column tile t covers B adjacent kx columns, so
 // tiles t and t+1 share the 128-byte lines of a row when B*8 < 128: map
@@ -1054,6 +1090,7 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         const size_t stride = ykind ? (size_t)hcs : (size_t)hcs * ny;
         const size_t off = ykind ? (size_t)outer * ny * hcs + kx0 : (size_t)outer * hcs + kx0;
         DWHIP_GL float2* __restrict__ dst = gp(MODE == CM_ZOTF ? J.K : J.C) + off;
+        if (MODE == CM_YFWD_PSF && !psf_covers(outer, gp(J.st)->mid[2], J.nz, J.pP)) continue;
         StageGeo g;
         g.n = ykind ? ny : J.nz;
         g.npen = B;
@@ -1073,13 +1110,15 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
                 constexpr bool adjoint = MODE == CM_YFWD_IMG || MODE == CM_ZCONVJ;
                 const int right = ext_right(gp(J.st)->mid[ykind ? 1 : 2], ykind ? J.pN : J.pP, adjoint);
                 return WrapPencils<cnt>{gp(J.C) + off, stride, nb, nin, nd, g.n, right};
+            } else if constexpr (MODE == CM_YFWD_PSF || MODE == CM_ZOTF) {
+                return PsfPencils<cnt>{gp(J.C) + off, stride, nb, g.n, gp(J.st)->mid[ykind ? 1 : 2], ykind ? J.pN : J.pP};
             } else {
                 return ColPencils<cnt>{gp(J.C) + off, stride, nb, nin, !ykind && nb == B && nin == g.n};
             }
         };
         const auto gsrc = make_src();
         const ColPencils<cnt> gdst{dst, stride, nb, nout, !ykind && nb == B && nout == g.n};
-        if (MODE == CM_YFWD || MODE == CM_YFWD_IMG) {
+        if (MODE == CM_YFWD || MODE == CM_YFWD_IMG || MODE == CM_YFWD_PSF) {
             fft_tile<DWHIP_YMAXE, -1, true, DWHIP_RMAX_Y, false, false>(J.pyf, g, tid, lds, gp(J.tw), gsrc, gdst);
         } else if (MODE == CM_YINV || MODE == CM_YINV_IMG) {
             fft_tile<DWHIP_YMAXE, +1, true, DWHIP_RMAX_Y, false, false>(J.pyi, g, tid, lds, gp(J.tw), gsrc, gdst);
