@@ -578,6 +578,7 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     d.metric = prm->metric;
     d.bg_auto = prm->bg_auto;
     d.start_identity = prm->start != DWHIP_START_FLAT;
+    d.flat = !d.start_identity && !j->generic;
     d.niter = niter;
     d.iter_type = prm->iter_type;
     d.err_rel = prm->err_rel;
@@ -841,10 +842,12 @@ int dwhip_job_round(DwhipJob* j, bool full, hipStream_t s)
         return DWHIP_OK;
     }
     const DwhipTiles& t = j->tiles;
-    RCHK(dwhip_pass_x(XM_UPDATE, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
-    RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
-    RCHK(dwhip_pass_c(CM_ZCONV, j, j->bd, j->jd, t.ntile[KIND_Z], t.lds[KIND_Z], s));
-    RCHK(dwhip_pass_c(CM_YINV_IMG, j, j->bd, j->jd, t.ntile[KIND_YD], t.lds[KIND_YD], s));
+    if (!j->d.flat || j->host_iter > 0) {  // iteration 0 of a flat start has no transform
+        RCHK(dwhip_pass_x(XM_UPDATE, j, j->bd, j->jd, t.ntile[KIND_X], t.lds[KIND_X], s));
+        RCHK(dwhip_pass_c(CM_YFWD, j, j->bd, j->jd, t.ntile[KIND_Y], t.lds[KIND_Y], s));
+        RCHK(dwhip_pass_c(CM_ZCONV, j, j->bd, j->jd, t.ntile[KIND_Z], t.lds[KIND_Z], s));
+        RCHK(dwhip_pass_c(CM_YINV_IMG, j, j->bd, j->jd, t.ntile[KIND_YD], t.lds[KIND_YD], s));
+    }
     RCHK(dwhip_pass_x(XM_RATIO, j, j->bd, j->jd, t.ntile[KIND_XR], t.lds[KIND_XR], s));
     if (full) {
         RCHK(dwhip_pass_c(CM_YFWD_IMG, j, j->bd, j->jd, t.ntile[KIND_YF], t.lds[KIND_YF], s));
@@ -915,15 +918,20 @@ static int fixed_loop(DwhipJob* job, int niter, bool may_graph, hipStream_t s, h
         for (int k = 0; k < niter; ++k) RCHK(dwhip_job_round(job, job->d.rl || k + 1 < niter, s));
         return DWHIP_OK;
     }
-    const int nfull = mode == 2 ? 1 : (job->d.rl ? niter : niter - 1);
-    LoopCtx c{job, niter, mode == 1};
-    hipGraphExec_t exec = nullptr;
-    RCHK(dwhip_capture(loop_body, &c, &exec));
-    *exec_out = exec;
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < nfull && e == hipSuccess; ++k) e = hipGraphLaunch(exec, s);
-    if (e != hipSuccess) return dwhip_hip_fail(e, "hipGraphLaunch", __LINE__);
-    job->host_iter = mode == 2 ? niter : nfull;
+    // round 0 of a flat start has passes of its own number
+    const int first = mode == 1 && job->d.flat ? 1 : 0;
+    if (first) RCHK(dwhip_job_round(job, true, s));
+    const int nfull = mode == 2 ? 1 : (job->d.rl ? niter : niter - 1) - first;
+    if (nfull > 0) {
+        LoopCtx c{job, niter, mode == 1};
+        hipGraphExec_t exec = nullptr;
+        RCHK(dwhip_capture(loop_body, &c, &exec));
+        *exec_out = exec;
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < nfull && e == hipSuccess; ++k) e = hipGraphLaunch(exec, s);
+        if (e != hipSuccess) return dwhip_hip_fail(e, "hipGraphLaunch", __LINE__);
+    }
+    job->host_iter = mode == 2 ? niter : first + nfull;
     if (mode == 1 && !job->d.rl) RCHK(dwhip_job_round(job, false, s));
     return DWHIP_OK;
 }
@@ -1278,6 +1286,7 @@ int dwhip_fft3_device(float* vol, float* spec, int64_t nx, int64_t ny, int64_t n
     // point U0 at the caller's volume
     JobDev d2 = d;
     d2.U0 = vol;
+    d2.flat = 0;  // the passes of a loop's iteration 0 would do nothing
     hipError_t e = hipMemcpy(job.jd, &d2, sizeof(d2), hipMemcpyHostToDevice);
     const DwhipTiles& t = job.tiles;
     const size_t rowb = (size_t)d.hc * sizeof(float2), pitch = (size_t)d.hcs * sizeof(float2);

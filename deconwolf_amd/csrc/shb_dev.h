@@ -63,6 +63,10 @@ struct JobDev {
     int has_w;          // Bertero weights in use (bq > 0)
     int bg_auto;
     int start_identity; // start from start_img (or im) inserted, instead of flat
+    // 1: flat start.  Iteration 0's forward model of a constant is the constant
+    // times the PSF's sum, so its update, y, z and y-inverse passes do nothing
+    // and its ratio pass starts from that value
+    int flat;
     int niter;          // iterations requested (nIter, or maxiter for REL/ABS)
     int rl;             // 1: Richardson-Lucy (method_rl.c), 0: SHB (method_shb.c)
     // 1: the adjoint half runs on the image's rows and planes alone.  The SHB

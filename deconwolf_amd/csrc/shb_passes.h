@@ -389,7 +389,9 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             if (!any) return;
         }
         const int iter = (MODE == XM_UPDATE || MODE == XM_RATIO) ? st->iter : 0;
-        const bool inv = MODE == XM_RATIO || MODE == XM_WEIGHTS || MODE == XM_STORE ||
+        const bool flat0 = J.flat && iter == 0;
+        if (MODE == XM_UPDATE && flat0) return;
+        const bool inv = (MODE == XM_RATIO && !flat0) || MODE == XM_WEIGHTS || MODE == XM_STORE ||
                          (MODE == XM_UPDATE && iter > 0);
         const bool fwd = MODE != XM_WEIGHTS && MODE != XM_STORE;
         StageGeo g;
@@ -471,6 +473,18 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             __syncthreads();
         }
 
+        // the PSF's sum: the OTF's first value without its scale
+        const float psum = (MODE == XM_UPDATE && J.rl && J.has_w) || (MODE == XM_RATIO && flat0)
+                               ? ldg(gp(J.K)).x * (((float)J.nx * (float)J.ny) * (float)J.nz)
+                               : 0.f;
+        if (MODE == XM_RATIO && flat0) {
+            // y = H p of p = x_0 (SHB: not below bg), a constant
+            const float p0 = !J.rl && st->c0 < st->bg ? st->bg : st->c0;
+            const float y0 = p0 * psum;
+            for (int w = tid; w < nrows * h; w += XTHR) lds[w] = make_float2(y0, y0);
+            __syncthreads();
+        }
+
         // elementwise step on packed real pairs (elements 2n, 2n+1 of a row),
         // in natural order in LDS; loads of XCHUNK elements are issued together
         double acc = 0;
@@ -489,9 +503,6 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         // alpha of iterations k-1 and k (uniform)
         const double am1 = MODE == XM_UPDATE ? shb_alpha(iter - 1, J.alphamax) : 0.0;
         const double al = MODE == XM_UPDATE ? shb_alpha(iter, J.alphamax) : 0.0;
-        // the PSF's sum: the OTF's first value without its scale
-        const float psum =
-            MODE == XM_UPDATE && J.rl && J.has_w ? ldg(gp(J.K)).x * (((float)J.nx * (float)J.ny) * (float)J.nz) : 0.f;
         // the pruned ratio pass's tiles lie within one plane: its rows' y and z
         // come from the tile (no division per element)
         const bool plane_tile = EXT || (xmode_image_rows(MODE) && J.prune);
@@ -524,7 +535,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
 #pragma unroll
             for (int q = 0; q < XCHUNK; ++q) {
                 if (!FULL::value && w0 + q * XTHR >= nwork) continue;
-                if (inv) a[q] = lds[lix(w0 + q * XTHR)];
+                if (inv || MODE == XM_RATIO) a[q] = lds[lix(w0 + q * XTHR)];
                 if (MODE == XM_UPDATE) {
                     b[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Ukm1 + vi[q]));
                     if (!J.rl) c[q] = ldgs<XNT>(reinterpret_cast<const DWHIP_GL float2*>(Uk + vi[q]));
@@ -1080,6 +1091,8 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         const int t = (ykind && (int)gridDim.x == total) ? xcd_tile(t0, total) : t0;
         const JobDev& J = jobs[find_job(jobs, njobs, kind, t)];
         if (J.dev_stop && gp(J.st)->stop) continue;  // the stopping rule ended this job
+        if ((MODE == CM_YFWD || MODE == CM_ZCONV || MODE == CM_YINV_IMG) && J.flat && gp(J.st)->iter == 0)
+            continue;  // iteration 0 of a flat start has no transform
         const int lt = t - J.tile0[kind];
         const int hcs = J.hcs, ny = J.ny;
         const int B = ykind ? J.ycols : J.zcols;

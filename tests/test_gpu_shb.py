@@ -215,3 +215,25 @@ def test_shb_degenerate_shapes(shape, psfshape):
         o32, e32, _, _ = ref(im, k, niter=6, work=s.stats["work"])
         assert rel_l2(out, o32) <= 1e-5, (method, rel_l2(out, o32))
         np.testing.assert_allclose(s.err_trace, e32, rtol=1e-4)
+
+
+# a flat start's iteration 0 has no transform: its forward model is the constant
+# times the PSF's sum.  The counts at which the loop leaves it, PSFs that do not sum to 1, a start below bg (the first
+# extrapolation is clamped), both methods, against the float32 oracle.
+@pytest.mark.parametrize("niter", [1, 2, 3, 4])
+@pytest.mark.parametrize("method", [dw.METHOD_SHB, dw.METHOD_RL])
+@pytest.mark.parametrize("scale,bq,bg", [(1.0, 2, None), (2.5, 2, None), (0.5, 1, None), (1.0, 0, None), (1.0, 2, 400.0)])
+def test_flat_start(niter, method, scale, bq, bg):
+    print("flat start", niter, method, scale, bq, bg, flush=True)
+    im, k = case((13, 28, 40), (7, 9, 9), seed=31)
+    k = (k * np.float32(scale)).astype(np.float32)
+    s = dw.DwOpts(nIter=niter, iter_type=dw.ITER_FIXED, borderQuality=bq, method=method)
+    kw = {}
+    if bg is not None:
+        s.bg_auto, s.bg = 0, bg
+        kw = dict(bg_auto=0, bg=bg)
+    rl = method == dw.METHOD_RL
+    out = (dw.deconvolve_rl_hip if rl else dw.deconvolve_shb_hip)(im, k, s)
+    o32, e32, _, _ = (po.rl if rl else po.shb)(im, k, niter=niter, border_quality=bq, work=s.stats["work"], **kw)
+    assert rel_l2(out, o32) <= 1e-5
+    np.testing.assert_allclose(s.err_trace, e32, rtol=1e-4)
