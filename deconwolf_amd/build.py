@@ -26,6 +26,8 @@ N_CMODES = 10
 # modes compiled for extended jobs too (xmode_has_ext, cmode_has_ext)
 EXT_XMODES = (1, 2, 3, 4)
 EXT_CMODES = (0, 1, 3, 4, 7, 8)
+# y modes, compiled for the small workgroups too
+Y_CMODES = (0, 1, 7, 8, 9)
 
 # -packed-fp32-ops: no packed FP32 instructions in device code.  The host
 # pass of hipcc warns that it does not know the feature; that is harmless.
@@ -54,6 +56,10 @@ def units():
         u.append(("k_colpass.hip", ["-DCMODE=%d" % m], "k_colpass_%d.o" % m))
     for m in EXT_CMODES:
         u.append(("k_colpass.hip", ["-DCMODE=%d" % m, "-DPASS_EXT"], "k_colpass_e%d.o" % m))
+    for m in Y_CMODES:
+        u.append(("k_colpass.hip", ["-DCMODE=%d" % m, "-DPASS_YSMALL"], "k_colpass_s%d.o" % m))
+        if m in EXT_CMODES:
+            u.append(("k_colpass.hip", ["-DCMODE=%d" % m, "-DPASS_EXT", "-DPASS_YSMALL"], "k_colpass_se%d.o" % m))
     u.append(("k_misc.hip", [], "k_misc.o"))
     u.append(("k_output.hip", [], "k_output.o"))
     u.append(("k_bw.hip", [], "k_bw.o"))

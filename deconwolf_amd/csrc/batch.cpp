@@ -113,6 +113,7 @@ struct Table {
     int n = 0;
     size_t lds[KIND_N] = {};
     int ntile[KIND_N] = {};
+    bool ysmall = false;  // every job's y tiles fit the small workgroups
     std::vector<EngJob*> jobs;
     BatchDev* bd() const { return (BatchDev*)dev; }
     JobDev* jd() const { return (JobDev*)(dev + 64); }
@@ -185,7 +186,9 @@ int table_build(Table* t, const std::vector<EngJob*>& jobs, hipStream_t s)
         t->ntile[k] = 0;
         t->lds[k] = 0;
     }
+    t->ysmall = true;
     for (int i = 0; i < t->n; ++i) {
+        t->ysmall = t->ysmall && jobs[i]->j.tiles.ysmall;
         jh[i] = jobs[i]->j.d;
         jh[i].dev_stop = dev_stop_job(jobs[i]) ? 1 : 0;
         for (int k = 0; k < KIND_N; ++k) {
@@ -207,7 +210,7 @@ int table_pass(const Table& t, bool xkind, int mode, hipStream_t s)
     if (t.n == 0 || t.ntile[kind] == 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
     hipError_t e = xkind ? dwhip_launch_xpass(mode, 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s)
-                         : dwhip_launch_colpass(mode, 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
+                         : dwhip_launch_colpass(mode, t.ysmall ? PASS_V_YSMALL : 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
     if (slot >= 0) {
         double by = 0;
         for (EngJob* j : t.jobs) by += dwhip_pass_bytes(xkind ? 1 : 0, mode, j->j.d, j->j.host_iter);

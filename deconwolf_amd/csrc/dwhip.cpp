@@ -341,7 +341,9 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
     const int hc = h + 1;
     t->xrows = std::max(1, std::min(DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / h));
     // a column tile holds B pencils of n complex values in LDS
-    const int ylim = std::min(DWHIP_YMAXE * DWHIP_CTHR, (int)(DWHIP_MAX_LDS_BYTES / sizeof(float2)));
+    t->ysmall = ny * DWHIP_YCOLS_LINE <= DWHIP_YMAXE * DWHIP_YTHR_SMALL;
+    const int ylim = std::min(DWHIP_YMAXE * (t->ysmall ? DWHIP_YTHR_SMALL : DWHIP_CTHR),
+                              (int)(DWHIP_MAX_LDS_BYTES / sizeof(float2)));
     const int zlim = std::min(DWHIP_ZMAXE * DWHIP_ZTHR, (int)(DWHIP_MAX_LDS_BYTES / sizeof(float2)));
     t->ycols = std::max(1, std::min(64, pow2_floor(ylim / ny)));
     t->zcols = std::max(1, std::min(64, pow2_floor(zlim / nz)));
@@ -784,7 +786,7 @@ int dwhip_pass_x(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 {
     if (ntile <= 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    hipError_t e = dwhip_launch_xpass(mode, j->ext && bd != j->obd, bd, jd, ntile, lds, s);
+    hipError_t e = dwhip_launch_xpass(mode, j->ext && bd != j->obd ? PASS_V_EXT : 0, bd, jd, ntile, lds, s);
     if (slot >= 0) dwhip_prof_end(s, slot, mode, dwhip_pass_bytes(1, mode, j->d, (int)host_iter(j, mode)));
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "x pass", __LINE__);
 }
@@ -794,7 +796,8 @@ int dwhip_pass_c(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 {
     if (ntile <= 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    hipError_t e = dwhip_launch_colpass(mode, j->ext && bd != j->obd, bd, jd, ntile, lds, s);
+    const int variant = (j->ext && bd != j->obd ? PASS_V_EXT : 0) | (j->tiles.ysmall ? PASS_V_YSMALL : 0);
+    hipError_t e = dwhip_launch_colpass(mode, variant, bd, jd, ntile, lds, s);
     if (slot >= 0) dwhip_prof_end(s, slot, 7 + mode, dwhip_pass_bytes(0, mode, j->d, 0));
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "column pass", __LINE__);
 }

@@ -253,12 +253,21 @@ DECL_LAUNCH(dwhip_launch_ce3)
 DECL_LAUNCH(dwhip_launch_ce4)
 DECL_LAUNCH(dwhip_launch_ce7)
 DECL_LAUNCH(dwhip_launch_ce8)
+DECL_LAUNCH(dwhip_launch_cs0)
+DECL_LAUNCH(dwhip_launch_cs1)
+DECL_LAUNCH(dwhip_launch_cs7)
+DECL_LAUNCH(dwhip_launch_cs8)
+DECL_LAUNCH(dwhip_launch_cs9)
+DECL_LAUNCH(dwhip_launch_cse0)
+DECL_LAUNCH(dwhip_launch_cse1)
+DECL_LAUNCH(dwhip_launch_cse7)
+DECL_LAUNCH(dwhip_launch_cse8)
 
 extern "C" {
 
 typedef hipError_t (*pass_launch)(const BatchDev*, const JobDev*, int, size_t, hipStream_t);
 
-hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+hipError_t dwhip_launch_xpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
                               hipStream_t s)
 {
     static_assert(XM_PSF == 0 && XM_STORE == 6, "X modes 0..6");
@@ -266,21 +275,28 @@ hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDe
         {dwhip_launch_x0, dwhip_launch_x1, dwhip_launch_x2, dwhip_launch_x3, dwhip_launch_x4, dwhip_launch_x5,
          dwhip_launch_x6},
         {nullptr, dwhip_launch_xe1, dwhip_launch_xe2, dwhip_launch_xe3, dwhip_launch_xe4, nullptr, nullptr}};
-    if (mode < 0 || mode > 6 || !f[ext ? 1 : 0][mode]) return hipErrorInvalidValue;
-    return f[ext ? 1 : 0][mode](bd, jobs, grid, lds, s);
+    const int v = variant & PASS_V_EXT;
+    if (mode < 0 || mode > 6 || !f[v][mode]) return hipErrorInvalidValue;
+    return f[v][mode](bd, jobs, grid, lds, s);
 }
 
-hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
+hipError_t dwhip_launch_colpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds,
                                 hipStream_t s)
 {
     static_assert(CM_YFWD == 0 && CM_YFWD_PSF == 9 && DWHIP_N_CMODES == 10, "column modes 0..9");
-    static const pass_launch f[2][DWHIP_N_CMODES] = {
+    static const pass_launch f[4][DWHIP_N_CMODES] = {
         {dwhip_launch_c0, dwhip_launch_c1, dwhip_launch_c2, dwhip_launch_c3, dwhip_launch_c4, dwhip_launch_c5,
          dwhip_launch_c6, dwhip_launch_c7, dwhip_launch_c8, dwhip_launch_c9},
         {dwhip_launch_ce0, dwhip_launch_ce1, nullptr, dwhip_launch_ce3, dwhip_launch_ce4, nullptr, nullptr,
-         dwhip_launch_ce7, dwhip_launch_ce8, nullptr}};
-    if (mode < 0 || mode >= DWHIP_N_CMODES || !f[ext ? 1 : 0][mode]) return hipErrorInvalidValue;
-    return f[ext ? 1 : 0][mode](bd, jobs, grid, lds, s);
+         dwhip_launch_ce7, dwhip_launch_ce8, nullptr},
+        {dwhip_launch_cs0, dwhip_launch_cs1, nullptr, nullptr, nullptr, nullptr, nullptr, dwhip_launch_cs7,
+         dwhip_launch_cs8, dwhip_launch_cs9},
+        {dwhip_launch_cse0, dwhip_launch_cse1, nullptr, nullptr, nullptr, nullptr, nullptr, dwhip_launch_cse7,
+         dwhip_launch_cse8, nullptr}};
+    if (mode < 0 || mode >= DWHIP_N_CMODES) return hipErrorInvalidValue;
+    const int v = cmode_is_y(mode) ? variant : variant & PASS_V_EXT;
+    if (v < 0 || v > 3 || !f[v][mode]) return hipErrorInvalidValue;
+    return f[v][mode](bd, jobs, grid, lds, s);
 }
 
 hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s)

@@ -45,6 +45,14 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #ifndef DWHIP_CTHR
 #define DWHIP_CTHR 1024  // threads per workgroup, Y passes (long pencils)
 #endif
+// Y workgroups where a tile of 16 columns (whole 128-byte lines) fits in
+// DWHIP_YMAXE values for each of half the threads: two workgroups per CU, one's
+// loads beside the other's transform.  y passes of 810 x 640 x 90: 94-103 us
+// with 1024 threads, 79-88 with 512; of 512 x 512 x 64: 42-45, 37-40.  Longer
+// pencils would leave 8 columns, half lines: 1250 x 1215 x 140 takes 383 us with
+// 1024 threads and 16 columns, 522 with 512 and 8.
+#define DWHIP_YTHR_SMALL 512
+#define DWHIP_YCOLS_LINE 16
 #ifndef DWHIP_ZTHR
 #define DWHIP_ZTHR 512   // threads per workgroup, Z passes
 #endif
@@ -73,9 +81,12 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #endif
 
 extern "C" {
-// ext: 1 launches the kernels of extended jobs (a table holds one kind)
-hipError_t dwhip_launch_xpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
-hipError_t dwhip_launch_colpass(int mode, int ext, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
+// variant: bits; PASS_V_EXT launches the kernels of extended jobs (a table holds
+// one kind), PASS_V_YSMALL y workgroups of DWHIP_YTHR_SMALL threads (every tile of
+// the table then fits them; the larger workgroups take any tile)
+enum { PASS_V_EXT = 1, PASS_V_YSMALL = 2 };
+hipError_t dwhip_launch_xpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
+hipError_t dwhip_launch_colpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
 hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s);
 hipError_t dwhip_launch_start(const JobDev* jobs, int j, int grid, hipStream_t s);
 hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int njobs, int advance, hipStream_t s);

@@ -1051,15 +1051,16 @@ __device__ __forceinline__ int xcd_tile(int b, int G)
     return x * q + min(x, r) + k;
 }
 
-template <int MODE>
+// threads of a column workgroup; YS: the small y workgroups
+template <int MODE, bool YS>
 constexpr int col_threads()
 {
-    return cmode_is_y(MODE) ? CTHR : ZTHR;
+    return cmode_is_y(MODE) ? (YS ? DWHIP_YTHR_SMALL : CTHR) : ZTHR;
 }
 
 // waves per SIMD the column kernels are compiled for (the VGPR budget):
-// Y tiles (1024 threads, up to 159 KiB of LDS, one per CU) need 4 and stay
-// within 128 VGPRs; Z tiles (512 threads, 10 values each, 35 KiB for
+// Y tiles (1024 threads, up to 159 KiB of LDS, one per CU; or 512 threads, two
+// per CU) need 4 and stay within 128 VGPRs; Z tiles (512 threads, 10 values each, 35 KiB for
 // nz = 140) fit 8 in 64 VGPRs, four workgroups per CU
 #ifndef DWHIP_Y_WAVES
 #define DWHIP_Y_WAVES 4
@@ -1073,15 +1074,15 @@ constexpr int col_waves()
     return cmode_is_y(MODE) ? DWHIP_Y_WAVES : DWHIP_Z_WAVES;
 }
 
-template <int MODE, bool EXT>
-__global__ __launch_bounds__(col_threads<MODE>()) __attribute__((amdgpu_waves_per_eu(col_waves<MODE>())))
+template <int MODE, bool EXT, bool YS>
+__global__ __launch_bounds__((col_threads<MODE, YS>())) __attribute__((amdgpu_waves_per_eu(col_waves<MODE>())))
 void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
 {
     extern __shared__ float2 lds[];
     const int tid = threadIdx.x;
     constexpr int kind = cmode_kind(MODE);
     constexpr bool ykind = cmode_is_y(MODE);
-    constexpr int NT = col_threads<MODE>();
+    constexpr int NT = col_threads<MODE, YS>();
     constexpr bool cnt = DWHIP_NT_COLS;
     static_assert(MODE >= 0 && MODE < DWHIP_N_CMODES, "column mode");
     const int total = bd->ntile[kind];
