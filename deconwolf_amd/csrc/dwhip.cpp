@@ -265,6 +265,7 @@ int dwhip_make_plan(int n, const std::vector<int>& r, FftPlanDev* p, std::vector
             }
         ns *= R;
     }
+    p->pad = p->nst > 1 ? plan_pad(n, r[0]) : 0;
     return ns == n || n == 1 ? DWHIP_OK : DWHIP_ERR_SIZE;
 }
 
@@ -339,7 +340,13 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
 {
     const int h = (int)(w[0] / 2), ny = (int)w[1], nz = (int)w[2];
     const int hc = h + 1;
-    t->xrows = std::max(1, std::min(DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / h));
+    // an x-row in LDS: its half spectrum while staged, or its values with the
+    // first exchange's pad of the forward or the inverse plan; three x
+    // workgroups share a CU's LDS
+    const std::vector<int> xr = pc && !pc->r[0].empty() ? pc->r[0] : dwhip_radices(h, 0);
+    const int xpad = xr.size() > 1 ? std::max(plan_pad(h, xr.front()), plan_pad(h, xr.back())) : 0;
+    const int xrow = std::max(hc, h + xpad) * (int)sizeof(float2);
+    t->xrows = std::max(1, std::min({DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / h, DWHIP_X_LDS_BYTES / xrow}));
     // a column tile holds B pencils of n complex values in LDS
     t->ysmall = ny * DWHIP_YCOLS_LINE <= DWHIP_YMAXE * DWHIP_YTHR_SMALL;
     const int ylim = std::min(DWHIP_YMAXE * (t->ysmall ? DWHIP_YTHR_SMALL : DWHIP_CTHR),
@@ -355,9 +362,7 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
     t->ntile[KIND_X] = (ny * nz + t->xrows - 1) / t->xrows;
     t->ntile[KIND_Y] = ((hc + t->ycols - 1) / t->ycols) * nz;
     t->ntile[KIND_Z] = ((hc + t->zcols - 1) / t->zcols) * ny;
-    // x tiles hold xrows rows of h values, or of hc values while the
-    // half-spectrum rows are staged
-    t->lds[KIND_X] = (size_t)t->xrows * (DWHIP_X_STAGE_LDS ? hc : h) * sizeof(float2);
+    t->lds[KIND_X] = (size_t)t->xrows * xrow;
     t->lds[KIND_Y] = (size_t)t->ycols * ny * sizeof(float2);
     t->lds[KIND_Z] = (size_t)t->zcols * nz * sizeof(float2);
     // the pruned y passes: all slabs until the job's image depth is known

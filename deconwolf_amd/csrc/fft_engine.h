@@ -36,7 +36,15 @@ struct FftPlanDev {
     int ns[DWHIP_MAX_STAGES];
     int twoff[DWHIP_MAX_STAGES];         // stage twiddles in the table (forward sign)
     uint32_t nsmagic[DWHIP_MAX_STAGES];  // fdiv magic of ns
+    int pad;  // rows: values added to a pencil's first exchange in LDS (plan_pad)
 };
+
+// Rows write their first stage's outputs at j*R + r: an even R puts the lanes
+// (consecutive j) on few LDS banks (16: all on two of them).  One unused value
+// after every R spreads them over all; odd radices do so by themselves.  x
+// passes of 512 x 512 x 64 (h = 256 = 16 * 16): update 113 -> 103 us, ratio 112
+// -> 95.
+__host__ __device__ constexpr int plan_pad(int n, int R1) { return R1 >= 8 && R1 % 2 == 0 ? n / R1 : 0; }
 
 // ---------------------------------------------------------------------------
 // complex helpers
@@ -343,6 +351,7 @@ struct StageGeo {
     int pstride;  // LDS pencil stride (rows layout)
     int nthr;
     int npshift;  // log2(npen) for column tiles
+    int pad;      // rows: the plan's pad (0: none) of the first exchange, pitch pstride + pad
 };
 
 // butterfly (pen, j) of work item w for a stage with nb butterflies per pencil
@@ -374,11 +383,25 @@ __device__ __forceinline__ int lds_in_step(const StageGeo& g, int nb)
 {
     return COLS ? nb * g.npen : nb;
 }
+// the second stage's input (FIRST: what the first stage wrote, padded by one
+// value after every ns, the first radix): element e at e + e / ns; jq = j / ns
+template <bool COLS, bool FIRST>
+__device__ __forceinline__ int lds_in2(const StageGeo& g, int w, int pen, int j, int jq)
+{
+    if (COLS || !FIRST) return lds_in<COLS>(g, w, pen, j);
+    return (int)__umul24((uint32_t)pen, (uint32_t)(g.pstride + g.pad)) + j + (g.pad ? jq : 0);
+}
+template <bool COLS, bool FIRST>
+__device__ __forceinline__ int lds_in2_step(const StageGeo& g, int nb, uint32_t nsmagic)
+{
+    if (COLS || !FIRST || !g.pad) return lds_in_step<COLS>(g, nb);
+    return nb + (int)fdiv((uint32_t)nb, nsmagic);
+}
 template <int R, bool COLS>
 __device__ __forceinline__ int lds_outR(const StageGeo& g, int w, int pen, int j)
 {
     return COLS ? w + (int)__umul24((uint32_t)j, (uint32_t)((R - 1) * g.npen))
-                : (int)__umul24((uint32_t)pen, (uint32_t)g.pstride) + j * R;
+                : (int)__umul24((uint32_t)pen, (uint32_t)(g.pstride + g.pad)) + j * R + (g.pad ? j : 0);
 }
 template <bool COLS>
 __device__ __forceinline__ int lds_outR_step(const StageGeo& g)
@@ -491,14 +514,14 @@ __device__ __forceinline__ void stage_first(const StageGeo& g, int tid, Src src,
 }
 
 // middle stage: LDS -> twiddle -> DFT -> LDS (in place, two barriers)
-template <int R, int MB, int DIR, bool COLS>
+template <int R, int MB, int DIR, bool COLS, bool FIRST>
 __device__ __forceinline__ void stage_mid(const StageGeo& g, int tid, float2* lds, int ns, uint32_t nsmagic,
                                           TwPtr __restrict__ tw)
 {
     const int nb = g.n / R;
     const uint32_t nbm = fdiv_magic((uint32_t)nb);
     const int total = nb * g.npen;
-    const int istep = lds_in_step<COLS>(g, nb);
+    const int istep = lds_in2_step<COLS, FIRST>(g, nb, nsmagic);
     float2 v[MB][R];
 #pragma unroll
     for (int q = 0; q < MB; ++q) {
@@ -506,7 +529,7 @@ __device__ __forceinline__ void stage_mid(const StageGeo& g, int tid, float2* ld
         if (w < total) {
             int pen, j;
             bfly_of<COLS>(g, w, nb, nbm, pen, j);
-            const float2* in = lds + lds_in<COLS>(g, w, pen, j);
+            const float2* in = lds + lds_in2<COLS, FIRST>(g, w, pen, j, (int)fdiv((uint32_t)j, nsmagic));
 #pragma unroll
             for (int r = 0; r < R; ++r) v[q][r] = in[r * istep];
         }
@@ -533,14 +556,16 @@ __device__ __forceinline__ void stage_mid(const StageGeo& g, int tid, float2* ld
 
 // last stage (ns = n/R, so the outputs of butterfly j are j + r*nb):
 // LDS -> twiddle -> DFT -> Dst
-template <int R, int MB, int DIR, bool COLS, bool SYNC, class Dst>
+template <int R, int MB, int DIR, bool COLS, bool SYNC, bool FIRST, class Dst>
 __device__ __forceinline__ void stage_last(const StageGeo& g, int tid, const float2* lds, TwPtr __restrict__ tw,
                                            Dst dst)
 {
     const int nb = g.n / R;
     const uint32_t nbm = fdiv_magic((uint32_t)nb);
     const int total = nb * g.npen;
-    const int istep = lds_in_step<COLS>(g, nb);
+    // FIRST: the second of two stages (nb is the first radix, so that element
+    // j + r * nb is padded by r)
+    const int istep = !COLS && FIRST && g.pad ? nb + 1 : lds_in_step<COLS>(g, nb);
     float2 v[MB][R];
 #pragma unroll
     for (int q = 0; q < MB; ++q) {
@@ -548,7 +573,7 @@ __device__ __forceinline__ void stage_last(const StageGeo& g, int tid, const flo
         if (w < total) {
             int pen, j;
             bfly_of<COLS>(g, w, nb, nbm, pen, j);
-            const float2* in = lds + lds_in<COLS>(g, w, pen, j);
+            const float2* in = lds + lds_in2<COLS, FIRST>(g, w, pen, j, 0);
 #pragma unroll
             for (int r = 0; r < R; ++r) v[q][r] = in[r * istep];
         }
@@ -712,26 +737,26 @@ __device__ __forceinline__ void run_first(int R, const StageGeo& g, int tid, Src
     }
 }
 
-template <int MAXE, int DIR, bool COLS, int RMAX>
+template <int MAXE, int DIR, bool COLS, int RMAX, bool FIRST>
 __device__ __forceinline__ void run_mid(int R, const StageGeo& g, int tid, float2* lds, int ns, uint32_t nsmagic,
                                         TwPtr __restrict__ tw)
 {
     switch (R) {
 #define CASE(RR) \
-    case RR: if constexpr (radix_ok(RMAX, RR)) { stage_mid<RR, mb_for(MAXE, RR), DIR, COLS>(g, tid, lds, ns, nsmagic, tw); } break;
+    case RR: if constexpr (radix_ok(RMAX, RR)) { stage_mid<RR, mb_for(MAXE, RR), DIR, COLS, FIRST>(g, tid, lds, ns, nsmagic, tw); } break;
         DWHIP_FOR_RADICES(CASE)
 #undef CASE
     default: break;
     }
 }
 
-template <int MAXE, int DIR, bool COLS, int RMAX, bool SYNC, class Dst>
+template <int MAXE, int DIR, bool COLS, int RMAX, bool SYNC, bool FIRST, class Dst>
 __device__ __forceinline__ void run_last(int R, const StageGeo& g, int tid, const float2* lds,
                                          TwPtr __restrict__ tw, Dst dst)
 {
     switch (R) {
 #define CASE(RR) \
-    case RR: if constexpr (radix_ok(RMAX, RR)) { stage_last<RR, mb_for(MAXE, RR), DIR, COLS, SYNC>(g, tid, lds, tw, dst); } break;
+    case RR: if constexpr (radix_ok(RMAX, RR)) { stage_last<RR, mb_for(MAXE, RR), DIR, COLS, SYNC, FIRST>(g, tid, lds, tw, dst); } break;
         DWHIP_FOR_RADICES(CASE)
 #undef CASE
     default: break;
@@ -770,8 +795,8 @@ __device__ __forceinline__ void run_mids(const FftPlanDev& p, const StageGeo& g,
     // At most four stages: straight-line code, so that the register
     // allocator sees disjoint stage bodies (a loop around the radix switch
     // makes their live ranges overlap).
-    if (p.nst > 2) run_mid<MAXE, DIR, COLS, RMAX>(p.radix[1], g, tid, lds, p.ns[1], p.nsmagic[1], tw + p.twoff[1]);
-    if (p.nst > 3) run_mid<MAXE, DIR, COLS, RMAX>(p.radix[2], g, tid, lds, p.ns[2], p.nsmagic[2], tw + p.twoff[2]);
+    if (p.nst > 2) run_mid<MAXE, DIR, COLS, RMAX, true>(p.radix[1], g, tid, lds, p.ns[1], p.nsmagic[1], tw + p.twoff[1]);
+    if (p.nst > 3) run_mid<MAXE, DIR, COLS, RMAX, false>(p.radix[2], g, tid, lds, p.ns[2], p.nsmagic[2], tw + p.twoff[2]);
 }
 
 // Src -> transform -> Dst.  The LDS must be free on entry.  SRC_LDS: Src
@@ -800,7 +825,11 @@ __device__ __forceinline__ void fft_tile(const FftPlanDev& p, const StageGeo& g,
     run_first<MAXE, DIR, COLS, RMAX, SRC_LDS>(p.radix[0], g, tid, src, lds);
     __syncthreads();
     run_mids<MAXE, DIR, COLS, RMAX>(p, g, tid, lds, tw);
-    run_last<MAXE, DIR, COLS, RMAX, DST_LDS>(p.radix[p.nst - 1], g, tid, lds, tw + p.twoff[p.nst - 1], dst);
+    // rows tell the second of two stages apart (its input is padded)
+    if (!COLS && p.nst == 2)
+        run_last<MAXE, DIR, COLS, RMAX, DST_LDS, true>(p.radix[1], g, tid, lds, tw + p.twoff[1], dst);
+    else
+        run_last<MAXE, DIR, COLS, RMAX, DST_LDS, false>(p.radix[p.nst - 1], g, tid, lds, tw + p.twoff[p.nst - 1], dst);
 }
 
 // Src -> transform (plan a, DIR1) -> op -> transform (plan b, DIR2) -> Dst,
@@ -833,7 +862,7 @@ __device__ __forceinline__ void fft_pair_tile(const FftPlanDev& a, const FftPlan
             run_mids<MAXE, DIR1, COLS, RMAX>(a, g, tid, lds, tw);                                          \
             stage_junction<RR, MB, DIR1, DIR2, COLS, PF>(g, tid, lds, tw + a.twoff[a.nst - 1], op, pf);    \
             run_mids<MAXE, DIR2, COLS, RMAX>(b, g, tid, lds, tw);                                          \
-            run_last<MAXE, DIR2, COLS, RMAX, false>(b.radix[b.nst - 1], g, tid, lds, tw + b.twoff[b.nst - 1], dst); \
+            run_last<MAXE, DIR2, COLS, RMAX, false, false>(b.radix[b.nst - 1], g, tid, lds, tw + b.twoff[b.nst - 1], dst); \
         }                                                                                                  \
         break;
         DWHIP_FOR_RADICES(CASE)

@@ -71,6 +71,9 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #ifndef DWHIP_ZMAXE
 #define DWHIP_ZMAXE 10   // Z passes: short pencils, many waves per SIMD
 #endif
+// LDS of an x tile: a third of the CU's 160 KiB less the static part, in the
+// 1280-byte units LDS is handed out in
+#define DWHIP_X_LDS_BYTES (42 * 1280 - 64)
 #ifndef DWHIP_XROWS_MAX
 #define DWHIP_XROWS_MAX 64  // rows per X tile at most
 #endif

@@ -326,14 +326,15 @@ __host__ __device__ constexpr bool x_fixed_mode(int mode)
 // x-row transform of a tile with plan p, or with the compile-time plan
 // (FR1, FR2) when FR1 > 0 (p then gives only the stage twiddle offsets)
 template <int FR1, int FR2, int DIR, bool SRC_LDS, bool DST_LDS, class Src, class Dst>
-__device__ __forceinline__ void x_fft(const FftPlanDev& p, const StageGeo& g, int tid, float2* lds, TwPtr __restrict__ tw,
+__device__ __forceinline__ void x_fft(const FftPlanDev& p, StageGeo g, int tid, float2* lds, TwPtr __restrict__ tw,
                                       Src src, Dst dst)
 {
+    g.pad = p.pad;
     if constexpr (FR1 > 0) {
         constexpr int RA = DIR < 0 ? FR1 : FR2, RB = DIR < 0 ? FR2 : FR1;
         stage_first<RA, mb_for(DWHIP_XMAXE, RA), DIR, false, SRC_LDS>(g, tid, src, lds);
         __syncthreads();
-        stage_last<RB, mb_for(DWHIP_XMAXE, RB), DIR, false, DST_LDS>(g, tid, lds, tw + p.twoff[1], dst);
+        stage_last<RB, mb_for(DWHIP_XMAXE, RB), DIR, false, DST_LDS, true>(g, tid, lds, tw + p.twoff[1], dst);
     } else {
         fft_tile<DWHIP_XMAXE, DIR, false, DWHIP_RMAX_X, SRC_LDS, DST_LDS>(p, g, tid, lds, tw, src, dst);
     }
@@ -400,6 +401,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         g.pstride = h;
         g.nthr = XTHR;
         g.npshift = 0;
+        g.pad = 0;
         const uint32_t hmagic = fdiv_magic((uint32_t)h);
         const DWHIP_GL float2* __restrict__ C = gp(J.C);
         TwPtr __restrict__ rtw = gp(J.rtw);
@@ -1111,6 +1113,7 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         g.pstride = 0;
         g.nthr = NT;
         g.npshift = __ffs(B) - 1;  // B is a power of two
+        g.pad = 0;
         // elements read (i < nin) and written (i < nout) along the pencil
         const int nd = EXT ? (ykind ? J.uy : J.uz) : g.n;  // data values along the pencil
         const int nin = (MODE == CM_YFWD_IMG && J.prune) ? J.N : (MODE == CM_ZCONVJ && J.prune) ? J.P

@@ -141,11 +141,11 @@ int dwhip_work_size(int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN, int
  * src/fft.c:135-172,206-319).  dwhip_plan_tune times, axis by axis, the
  * radix orders and tile shapes the kernels can run for the transform size
  * work (as dwhip_work_size returns it) against the rule planner's plan,
- * keeps a candidate only when it is more than 3 % faster, and stores the
+ * keeps a candidate only when it is more than 6 % faster, and stores the
  * plan in the process's plan cache and its file; retune != 0 measures a
  * size already cached.  tuned_ms / rule_ms (may be NULL) receive the
  * summed pass times of the chosen and of the rule's plan.  The cache file
- * is $DWHIP_PLAN_CACHE, else $HOME/.config/deconwolf/dwhip_plans_gfx950.txt
+ * is $DWHIP_PLAN_CACHE, else $HOME/.config/deconwolf/dwhip_plans_gfx950_k2.txt
  * (where deconwolf keeps its FFTW wisdom) when $HOME/.config exists;
  * dwhip_plan_cache_path sets another ("" for none, NULL for the default)
  * and loads it.  dwhip_plan_get writes the plan a job of size work uses:

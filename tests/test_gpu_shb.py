@@ -66,6 +66,16 @@ def test_fft3_forward_inverse(shape):
     assert err2 < 2e-6, err2
 
 
+# x rows whose first exchange in LDS is padded (an even first radix from 8 on) in
+# the forward transform, the inverse or both: two, three and four stages, one
+# row, a last tile that is not full
+@pytest.mark.parametrize("nx", [128, 256, 320, 360, 480, 512, 640, 896, 1008, 1440, 2048, 4096, 10080])
+@pytest.mark.parametrize("rows", [1, 67])
+def test_fft3_padded_rows(nx, rows):
+    print("fft3 padded rows", nx, rows, flush=True)
+    test_fft3_forward_inverse((1, rows, nx) if rows == 1 else (1, 70, nx))
+
+
 def test_fft3_matches_oracle_fft():
     rng = np.random.default_rng(3)
     vol = rng.standard_normal((7, 9, 10)).astype(np.float32)
