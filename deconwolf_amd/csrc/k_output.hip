@@ -16,6 +16,8 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "dwhip.h"
 #include "dwhip_internal.h"
 
@@ -46,18 +48,48 @@ struct OutStats {
     unsigned long long nbg;
 };
 
-__global__ __launch_bounds__(OTHR) void k_out_stats(const float* __restrict__ v, int64_t n, float bg,
+// Both kernels stream the volume once and are bound by its bytes: four values
+// per load (16-byte aligned volumes; others one by one), OUT_Q loads in flight
+// per thread.  1024 x 1024 x 60: statistics 131 -> 63 us, conversion 94 -> 63.
+#define OUT_Q 4
+struct alignas(8) U16x4 {
+    uint16_t v[4];
+};
+
+__global__ __launch_bounds__(OTHR) void k_out_stats(const float* __restrict__ v, int64_t n, int64_t n4, float bg,
                                                     OutStats* __restrict__ st)
 {
     __shared__ unsigned int smax[OTHR / 64];
     __shared__ unsigned long long scnt[OTHR / 64];
     unsigned int mk = 0;
     unsigned long long cnt = 0;
-    for (int64_t i = (int64_t)blockIdx.x * OTHR + threadIdx.x; i < n; i += (int64_t)gridDim.x * OTHR) {
-        const float x = v[i];
+    auto take = [&](float x) {
         if (x == x) mk = max(mk, float_key(x));
         cnt += (x == bg);
+    };
+    const int64_t S = (int64_t)gridDim.x * OTHR, i0 = (int64_t)blockIdx.x * OTHR + threadIdx.x;
+    const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
+    int64_t i = i0;
+    for (; i + (OUT_Q - 1) * S < n4; i += OUT_Q * S) {
+        float4 x[OUT_Q];
+#pragma unroll
+        for (int q = 0; q < OUT_Q; ++q) x[q] = v4[i + q * S];
+#pragma unroll
+        for (int q = 0; q < OUT_Q; ++q) {
+            take(x[q].x);
+            take(x[q].y);
+            take(x[q].z);
+            take(x[q].w);
+        }
     }
+    for (; i < n4; i += S) {
+        const float4 x = v4[i];
+        take(x.x);
+        take(x.y);
+        take(x.z);
+        take(x.w);
+    }
+    for (i = 4 * n4 + i0; i < n; i += S) take(v[i]);
     for (int o = 32; o > 0; o >>= 1) {
         mk = max(mk, __shfl_xor(mk, o));
         cnt += __shfl_xor(cnt, o);
@@ -96,17 +128,38 @@ __device__ __forceinline__ uint16_t to_u16(float x, float scaling)
 }
 
 template <int MODE>
-__global__ __launch_bounds__(OTHR) void k_to_u16(const float* __restrict__ v, int64_t n, float scaling,
+__global__ __launch_bounds__(OTHR) void k_to_u16(const float* __restrict__ v, int64_t n, int64_t n4, float scaling,
                                                  uint16_t* __restrict__ out)
 {
-    for (int64_t i = (int64_t)blockIdx.x * OTHR + threadIdx.x; i < n; i += (int64_t)gridDim.x * OTHR)
-        out[i] = to_u16<MODE>(v[i], scaling);
+    const int64_t S = (int64_t)gridDim.x * OTHR, i0 = (int64_t)blockIdx.x * OTHR + threadIdx.x;
+    const float4* __restrict__ v4 = reinterpret_cast<const float4*>(v);
+    U16x4* __restrict__ o4 = reinterpret_cast<U16x4*>(out);
+    auto conv = [&](float4 x) {
+        return U16x4{{to_u16<MODE>(x.x, scaling), to_u16<MODE>(x.y, scaling), to_u16<MODE>(x.z, scaling),
+                      to_u16<MODE>(x.w, scaling)}};
+    };
+    int64_t i = i0;
+    for (; i + (OUT_Q - 1) * S < n4; i += OUT_Q * S) {
+        float4 x[OUT_Q];
+#pragma unroll
+        for (int q = 0; q < OUT_Q; ++q) x[q] = v4[i + q * S];
+#pragma unroll
+        for (int q = 0; q < OUT_Q; ++q) o4[i + q * S] = conv(x[q]);
+    }
+    for (; i < n4; i += S) o4[i] = conv(v4[i]);
+    for (i = 4 * n4 + i0; i < n; i += S) out[i] = to_u16<MODE>(v[i], scaling);
 }
 
 static int out_grid(int64_t n)
 {
-    const int64_t g = (n + OTHR - 1) / OTHR;
+    const int64_t g = (n + 4 * OTHR - 1) / (4 * OTHR);
     return (int)(g < 4096 ? (g > 0 ? g : 1) : 4096);
+}
+
+// values taken four at a time: all but the last few of an aligned volume
+static int64_t out_quads(const float* v, const uint16_t* out, int64_t n)
+{
+    return ((uintptr_t)v & 15) == 0 && ((uintptr_t)out & 7) == 0 ? n / 4 : 0;
 }
 
 extern "C" {
@@ -119,16 +172,21 @@ int dwhip_output_stats_device(const float* v, int64_t n, float bg, float* vmax, 
     hipStream_t s = (hipStream_t)stream;
     OutStats* d = nullptr;
     OutStats h;
-    hipError_t e = hipMalloc((void**)&d, sizeof(OutStats));
+    // from the stream-ordered pool (hipMalloc and hipFree wait for the device)
+    hipError_t e = hipMallocAsync((void**)&d, sizeof(OutStats), s);
     if (e != hipSuccess) return e == hipErrorOutOfMemory ? DWHIP_ERR_NOMEM : DWHIP_ERR_HIP;
     e = hipMemsetAsync(d, 0, sizeof(OutStats), s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_out_stats, dim3(out_grid(n)), dim3(OTHR), 0, s, v, n, bg, d);
+        // (every workgroup ends in two atomics on one line: a thousand at most)
+        hipLaunchKernelGGL(k_out_stats, dim3(std::min(out_grid(n), 1024)), dim3(OTHR), 0, s, v, n, out_quads(v, nullptr, n), bg, d);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, s);
+    {
+        const hipError_t f = hipFreeAsync(d, s);
+        if (e == hipSuccess) e = f;
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d);
     if (e != hipSuccess) return dwhip_hip_fail(e, "output statistics", __LINE__);
     // key 0 means every value was NaN
     if (vmax) *vmax = h.maxkey ? key_float(h.maxkey) : NAN;
@@ -145,12 +203,13 @@ int dwhip_to_u16_device(const float* v, int64_t n, float scaling, int mode, uint
     if (rc != DWHIP_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     const int g = out_grid(n);
+    const int64_t n4 = out_quads(v, out, n);
     if (mode == DWHIP_U16_ROUND)
-        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_ROUND>, dim3(g), dim3(OTHR), 0, s, v, n, scaling, out);
+        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_ROUND>, dim3(g), dim3(OTHR), 0, s, v, n, n4, scaling, out);
     else if (mode == DWHIP_U16_TRUNC)
-        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_TRUNC>, dim3(g), dim3(OTHR), 0, s, v, n, scaling, out);
+        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_TRUNC>, dim3(g), dim3(OTHR), 0, s, v, n, n4, scaling, out);
     else
-        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_RINT>, dim3(g), dim3(OTHR), 0, s, v, n, scaling, out);
+        hipLaunchKernelGGL(k_to_u16<DWHIP_U16_RINT>, dim3(g), dim3(OTHR), 0, s, v, n, n4, scaling, out);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "u16 conversion", __LINE__);
 }

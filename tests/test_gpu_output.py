@@ -119,3 +119,22 @@ def test_to_host_from_threads_and_streams():
         t.join()
     for i in range(4):
         assert np.all(got[i] == 3.0 * (i + 1))
+
+
+# lengths around a load of four values, a workgroup's and a grid's share, and
+# volumes that start off a 16-byte boundary (taken one value at a time)
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 4096 * 256 * 4 + 7])
+@pytest.mark.parametrize("shift", [0, 1, 2])
+def test_output_lengths_and_alignment(n, shift):
+    print("output length", n, shift, flush=True)
+    rng = np.random.default_rng(n + shift)
+    v = np.where(rng.random(n) < 0.4, 7.5, rng.uniform(-10, 4000, n)).astype(np.float32)
+    v[: min(n, EDGES.size)] = EDGES[: min(n, EDGES.size)]
+    buf = torch.zeros(n + 4, device=DEV)
+    t = buf[shift:shift + n]
+    t.copy_(torch.from_numpy(v))
+    vmax, nbg = output.stats(t, 7.5)
+    assert vmax == float(np.nanmax(v)) and nbg == int((v == np.float32(7.5)).sum())
+    for mode in (output.U16_ROUND, output.U16_TRUNC, output.U16_RINT):
+        a = output.to_u16(t, 1.7, mode)
+        np.testing.assert_array_equal(a, ref_u16(v, 1.7, mode))
