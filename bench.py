@@ -17,7 +17,7 @@ bytes per launch over its mean launch duration, both from HIP events
 around every launch on the stream it runs on.  After the timed steps come
 the c4 request stream (`served`), the c3 tiled image (`tiled`), a c5
 sample (`c5`: the four channels of one multi-channel field, engine against
-plain) and the c2 image at border quality 1 on the any-size path
+plain) and the c2 image at border quality 1 at deconwolf's exact size
 (`anysize`), each with its own rates; none of them is `value`.
 """
 import argparse
@@ -375,7 +375,7 @@ def run_anysize():
         best[n] = min(best.get(n, 1e9), time.perf_counter() - t0)
     it_ms = 1e3 * (best[13] - best[3]) / 10
     M, N, P = im.shape[2], im.shape[1], im.shape[0]
-    return {"workload": "c2 at border quality 1: 1024x1024x60, PSF 181x181x79, work size %s (any-size path)" %
+    return {"workload": "c2 at border quality 1: 1024x1024x60, PSF 181x181x79, work size %s (extended job)" %
                         "x".join(str(v) for v in s.stats["work"]),
             "job_3_iterations_s": best[3], "job_13_iterations_s": best[13], "ms_per_iteration": it_ms,
             "image_voxel_iter_per_s": M * N * P / (it_ms * 1e-3)}
@@ -395,7 +395,7 @@ def main():
                          "engine) and plain (one at a time); 0 skips it")
     ap.add_argument("--rate", type=float, default=20.0, help="Poisson arrival rate of the stream, jobs/s")
     ap.add_argument("--no-tiled", action="store_true", help="skip the c3 tiled run")
-    ap.add_argument("--no-anysize", action="store_true", help="skip the c2 border-quality-1 (any-size path) timing")
+    ap.add_argument("--no-anysize", action="store_true", help="skip the c2 border-quality-1 (exact size) timing")
     ap.add_argument("--c5-fields", type=int, default=1, help="fields of the c5 sample (4 channels each); 0 skips it")
     ap.add_argument("--engine-groups", type=int, default=ENGINE_GROUPS, choices=(1, 2),
                     help="job groups of the engine runs (2: two streams whose passes overlap)")
