@@ -163,7 +163,14 @@ void save_locked()
         if (e_ != hipSuccess) return dwhip_hip_fail(e_, #call, __LINE__); \
     } while (0)
 
-// Mean time (ms) of the passes of `axis` for plan c on the block mem.
+// The image a trial of size w deconvolves: half the transform along each axis.
+void trial_image(const int64_t* w, int64_t* m)
+{
+    for (int d = 0; d < 3; ++d) m[d] = std::max<int64_t>(1, w[d] / 2);
+}
+
+// Mean time (ms) of the passes of `axis` for plan c on the block mem: cap bytes
+// for the job, then its image.
 int time_axis(const Key& w, int method, const DwhipPlanChoice& c, int axis, void* mem, size_t cap, hipStream_t s,
               hipEvent_t e0, hipEvent_t e1, double* ms)
 {
@@ -174,11 +181,12 @@ int time_axis(const Key& w, int method, const DwhipPlanChoice& c, int axis, void
     dwhip_params_default(&prm, 2);
     prm.method = method;
     for (int d = 0; d < 3; ++d) prm.work[d] = w[d];
-    // the image and PSF are not read by the timed passes; the job sizes are
-    // those of a job whose work size is w
-    const float* none = reinterpret_cast<const float*>(mem);
-    int rc = dwhip_job_plan(&j, none, std::max<int64_t>(1, w[0] / 2), std::max<int64_t>(1, w[1] / 2),
-                            std::max<int64_t>(1, w[2] / 2), none, 1, 1, 1, &prm, nullptr);
+    // the ratio pass reads the image, which the job's block must not hold (the
+    // pass overwrites C); no timed pass reads the PSF
+    const float* im = reinterpret_cast<const float*>((const char*)mem + cap);
+    int64_t m[3];
+    trial_image(w.data(), m);
+    int rc = dwhip_job_plan(&j, im, m[0], m[1], m[2], im, 1, 1, 1, &prm, nullptr);
     if (rc != DWHIP_OK) return rc;
     if (j.bytes > cap) return DWHIP_ERR_NOMEM;
     rc = dwhip_job_bind(&j, mem, s);
@@ -231,12 +239,11 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
     dwhip_tile_config(wv, &rt);
     const int rule_tile[3] = {rt.xrows, rt.ycols, rt.zcols};
 
-    // one block for every candidate (the layout depends on the plan only
-    // through the twiddle table and the partial sums)
-    size_t cap = dwhip_job_bytes(wv, std::max<int64_t>(1, w[0] / 2), std::max<int64_t>(1, w[1] / 2),
-                                 std::max<int64_t>(1, w[2] / 2), 1, 1, 1, 2, 2) + ((size_t)4 << 20);
+    // one block for every candidate
+    size_t cap = 0, image = 0;
+    dwhip_plan_trial_block(wv, &cap, &image);
     void* mem = nullptr;
-    TCHK(hipMalloc(&mem, cap));
+    TCHK(hipMalloc(&mem, cap + image));
     hipStream_t s = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = DWHIP_OK;
@@ -244,6 +251,7 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
     if (he == hipSuccess) he = hipEventCreate(&e0);
     if (he == hipSuccess) he = hipEventCreate(&e1);
     if (he == hipSuccess) he = hipMemsetAsync(mem, 0, cap, s);
+    if (he == hipSuccess) he = hipMemsetD32Async((hipDeviceptr_t)((char*)mem + cap), 0x3f800000, image / sizeof(float), s);
     if (he != hipSuccess) rc = dwhip_hip_fail(he, "tuner set-up", __LINE__);
 
     DwhipPlanChoice cur;  // rule plan: empty lists, zero tiles
@@ -293,6 +301,16 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
 }
 
 }  // namespace
+
+// Bytes of a trial's block: the job's (the layout depends on the plan only
+// through the twiddle table and the partial sums), then its image's.
+extern "C" void dwhip_plan_trial_block(const int64_t* w, size_t* job, size_t* image)
+{
+    int64_t m[3];
+    trial_image(w, m);
+    *job = (dwhip_job_bytes(w, m[0], m[1], m[2], 1, 1, 1, 2, 2) + ((size_t)4 << 20) + 255) / 256 * 256;
+    *image = (size_t)m[0] * m[1] * m[2] * sizeof(float);
+}
 
 bool dwhip_plan_cached(const int64_t* w, DwhipPlanChoice* pc)
 {

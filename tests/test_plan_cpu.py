@@ -1,0 +1,79 @@
+"""Host-side plans without a GPU: what dwhip_job_plan lays out, read through a
+small program compiled against the library's internal header."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "deconwolf_amd", "csrc")
+HIPCC = "/opt/rocm/bin/hipcc" if os.path.exists("/opt/rocm/bin/hipcc") else shutil.which("hipcc")
+
+
+@pytest.fixture(scope="session")
+def probe(tmp_path_factory):
+    """run(body, rows): a C++ program that reads rows of integers into v[] and
+    runs `body` for each; its output lines as lists of integers."""
+    if not HIPCC:
+        pytest.skip("no hipcc")
+    d = tmp_path_factory.mktemp("plan")
+
+    def run(body, rows):
+        n = len(rows[0])
+        src = d / ("p%d.cpp" % (abs(hash(body)) % 10 ** 9))
+        exe = str(src)[:-4]
+        src.write_text("""
+#include <hip/hip_runtime.h>
+#include <stdio.h>
+#include "dwhip.h"
+#include "dwhip_internal.h"
+int main() {
+    dwhip_plan_cache_path("");
+    long long v[%d];
+    for (;;) {
+        for (int i = 0; i < %d; ++i) if (scanf("%%lld", &v[i]) != 1) return 0;
+        %s
+    }
+}""" % (n, n, body))
+        lib = os.path.join(ROOT, "deconwolf_amd", "libdwhip.so")
+        subprocess.run([HIPCC, "--cuda-host-only", "-O0", "-w", "-x", "hip", "-I" + os.path.join(ROOT, "include"),
+                        "-I" + CSRC, str(src), "-x", "none", lib, "-Wl,-rpath," + os.path.dirname(lib), "-o", exe],
+                       check=True)
+        out = subprocess.run([exe], input="\n".join(" ".join(map(str, r)) for r in rows), text=True,
+                             capture_output=True, check=True).stdout
+        return [[int(x) for x in line.split()] for line in out.splitlines()]
+    return run
+
+
+# smallest, odd-rowed, ordinary and large transform sizes of the fused passes
+FAST = [(2, 1, 1), (4, 3, 5), (64, 45, 21), (256, 256, 96), (810, 640, 90), (1250, 1215, 140), (4096, 27, 8)]
+
+
+def test_trial_image_lies_outside_the_job(probe):
+    """The planner's trial runs the ratio pass, which reads the job's image and
+    overwrites its spectrum: the image has memory of its own, behind the block
+    of every candidate (the layout of the smallest tiles is the largest)."""
+    body = """
+        int64_t w[3] = {v[0], v[1], v[2]};
+        size_t job = 0, image = 0;
+        dwhip_plan_trial_block(w, &job, &image);
+        const int64_t m[3] = {w[0] / 2, w[1] > 1 ? w[1] / 2 : 1, w[2] > 1 ? w[2] / 2 : 1};
+        size_t most = 0;
+        for (int x = 0; x <= 1; ++x) {
+            DwhipPlanChoice c;
+            if (x) c.xrows = c.ycols = c.zcols = 1;
+            DwhipJob j;
+            j.force_plan = &c;
+            dwhip_params p;
+            dwhip_params_default(&p, 2);
+            for (int d = 0; d < 3; ++d) p.work[d] = w[d];
+            const float* im = (const float*)(uintptr_t)256;
+            if (dwhip_job_plan(&j, im, m[0], m[1], m[2], im, 1, 1, 1, &p, nullptr) != DWHIP_OK) return 1;
+            if (j.bytes > most) most = j.bytes;
+        }
+        printf("%zu %zu %zu %lld\\n", job, image, most, (long long)(m[0] * m[1] * m[2] * 4));
+    """
+    for job, image, most, need in probe(body, FAST):
+        assert job % 256 == 0 and most <= job
+        assert image >= need
