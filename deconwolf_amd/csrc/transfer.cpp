@@ -87,6 +87,12 @@ extern "C" int dwhip_download(void* dst, const void* src, size_t bytes, void* st
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "download", __LINE__);
     }
+    if (s == hipStreamPerThread) {
+        // the handle names another stream in each thread: what is queued on
+        // this thread's is waited for here
+        e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return dwhip_hip_fail(e, "download", __LINE__);
+    }
     // as many threads as the machine has, this one among them; where one
     // cannot be started its chunks are taken here, after this thread's own
     const int n = std::max(1, std::min(kWorkers, (int)std::thread::hardware_concurrency()));
