@@ -112,7 +112,9 @@ __global__ __launch_bounds__(STHR) void k_stats_final(const JobDev* __restrict__
     if (tid != 0) return;
     vmin = smin[0];
     vsum = ssum[0];
-    vidx = sidx[0];
+    // a PSF without a value above -inf (NaN in all of it) has no maximum: its
+    // first value, as fim_argmax_max takes it (fim.c:269-332)
+    vidx = sidx[0] < 1e300 ? sidx[0] : 0;
     JobState* st = J.st;
     // bg_auto: bg = max(min(im), 1e-2)  (method_shb.c:108-117)
     float bg = J.bg_user;
