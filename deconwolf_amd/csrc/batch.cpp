@@ -314,8 +314,7 @@ int setup(dwhip_engine* E, const std::vector<EngJob*>& fresh)
     if (fast.empty()) return DWHIP_OK;
     RCHK(table_build(&E->tsetup, fast, s));
     for (int i = 0; i < (int)fast.size(); ++i) {
-        const JobDev& d = fast[i]->j.d;
-        ECHK(dwhip_launch_stats(E->tsetup.jd(), i, (int64_t)d.M * d.N * d.P, s));
+        ECHK(dwhip_launch_stats(E->tsetup.jd(), i, &fast[i]->j.d, s));
         ECHK(dwhip_launch_start(E->tsetup.jd(), i, 1024, s));
     }
     RCHK(table_pass(E->tsetup, true, XM_PSF, s));

@@ -818,7 +818,7 @@ int dwhip_job_setup(const DwhipJob* j, hipStream_t s)
 {
     if (j->generic) return dwhip_generic_setup(j, s);
     const DwhipTiles& t = j->tiles;
-    HIPCHK(dwhip_launch_stats(j->jd, 0, (int64_t)j->d.M * j->d.N * j->d.P, s));
+    HIPCHK(dwhip_launch_stats(j->jd, 0, &j->d, s));
     HIPCHK(dwhip_launch_start(j->jd, 0, 1024, s));
     // OTF: shifted PSF -> R2C -> K / (nx*ny*nz)
     {

@@ -287,7 +287,7 @@ int convolve(const DwhipJob* j, bool conj, hipStream_t s)
 // OTF, Bertero weights and start guess (method_shb.c:108-294).
 int dwhip_generic_setup(const DwhipJob* j, hipStream_t s)
 {
-    hipError_t e = dwhip_launch_stats(j->jd, 0, (int64_t)j->d.M * j->d.N * j->d.P, s);
+    hipError_t e = dwhip_launch_stats(j->jd, 0, &j->d, s);
     if (e == hipSuccess) e = dwhip_launch_start(j->jd, 0, 1024, s);
     if (e != hipSuccess) return dwhip_hip_fail(e, "any-size set-up", __LINE__);
     GCHK(elem(j, OP_PSF, s));

@@ -301,12 +301,19 @@ hipError_t dwhip_launch_colpass(int mode, int variant, const BatchDev* bd, const
     return f[v][mode](bd, jobs, grid, lds, s);
 }
 
-hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s)
+int dwhip_stat_blocks(const JobDev* d)
 {
-    // at least eight values per thread (their loads are issued together), and
-    // four workgroups per CU for a large image: 1024 x 1024 x 60 takes
-    // 63 us (113 with one per CU)
-    const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(DWHIP_STAT_BLOCKS, nvox / (8 * STHR)));
+    // at least eight values of the image or the PSF per thread (their loads are
+    // issued together), and four workgroups per CU for a large one: 1024 x 1024 x
+    // 60 takes 63 us (113 with one per CU).  Each leaves four doubles in C.
+    const int64_t n = std::max((int64_t)d->M * d->N * d->P, (int64_t)d->pM * d->pN * d->pP);
+    const int64_t room = (int64_t)d->hcs * d->ny * d->uz * (int64_t)sizeof(float2) / (4 * (int64_t)sizeof(double));
+    return (int)std::max<int64_t>(1, std::min({(int64_t)DWHIP_STAT_BLOCKS, room, n / (8 * STHR)}));
+}
+
+hipError_t dwhip_launch_stats(const JobDev* jobs, int j, const JobDev* d, hipStream_t s)
+{
+    const int nblk = dwhip_stat_blocks(d);
     hipLaunchKernelGGL(k_stats_partial, dim3(nblk), dim3(STHR), 0, s, jobs, j, nblk);
     hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(STHR), 0, s, jobs, j, nblk);
     return hipGetLastError();

@@ -90,7 +90,9 @@ extern "C" {
 enum { PASS_V_EXT = 1, PASS_V_YSMALL = 2 };
 hipError_t dwhip_launch_xpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
 hipError_t dwhip_launch_colpass(int mode, int variant, const BatchDev* bd, const JobDev* jobs, int grid, size_t lds, hipStream_t s);
-hipError_t dwhip_launch_stats(const JobDev* jobs, int j, int64_t nvox, hipStream_t s);
+// workgroups of the statistics of job d (host copy of its descriptor)
+int dwhip_stat_blocks(const JobDev* d);
+hipError_t dwhip_launch_stats(const JobDev* jobs, int j, const JobDev* d, hipStream_t s);
 hipError_t dwhip_launch_start(const JobDev* jobs, int j, int grid, hipStream_t s);
 hipError_t dwhip_launch_round_end(const BatchDev* bd, const JobDev* jobs, int njobs, int advance, hipStream_t s);
 hipError_t dwhip_launch_crop(const JobDev* jobs, int j, int k, float* out, int64_t nrows, hipStream_t s);

@@ -77,3 +77,26 @@ def test_trial_image_lies_outside_the_job(probe):
     for job, image, most, need in probe(body, FAST):
         assert job % 256 == 0 and most <= job
         assert image >= need
+
+
+# image and PSF: either larger, both small, a PSF longer than the period (bq 1)
+STATS = [(1, 1, 1, 1, 1, 1, 2), (40, 36, 1, 181, 181, 79, 2), (8, 8, 8, 63, 63, 63, 1), (64, 64, 8, 181, 181, 31, 1),
+         (1024, 1024, 60, 181, 181, 79, 2), (37, 23, 11, 9, 9, 7, 0), (5, 8, 2503, 3, 3, 5, 0)]
+
+
+def test_statistics_cover_the_psf_and_fit_the_spectrum(probe):
+    """The set-up statistics' grid follows the larger of image and PSF (both are
+    walked), and its partials, which lie in C, fit there."""
+    body = """
+        DwhipJob j;
+        dwhip_params p;
+        dwhip_params_default(&p, 2);
+        p.border_quality = v[6];
+        const float* im = (const float*)(uintptr_t)256;
+        if (dwhip_job_plan(&j, im, v[0], v[1], v[2], im, v[3], v[4], v[5], &p, nullptr) != DWHIP_OK) return 1;
+        printf("%d %zu\\n", dwhip_stat_blocks(&j.d), j.lay.K - j.lay.C);
+    """
+    for (M, N, P, pM, pN, pP, _), (blocks, room) in zip(STATS, probe(body, STATS)):
+        assert 1 <= blocks <= 1024 and 32 * blocks <= room
+        n = max(M * N * P, pM * pN * pP)
+        assert blocks in (1024, room // 32, max(1, n // 2048))
