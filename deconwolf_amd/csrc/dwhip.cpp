@@ -346,7 +346,7 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
     const std::vector<int> xr = pc && !pc->r[0].empty() ? pc->r[0] : dwhip_radices(h, 0);
     const int xpad = xr.size() > 1 ? std::max(plan_pad(h, xr.front()), plan_pad(h, xr.back())) : 0;
     const int xrow = std::max(hc, h + xpad) * (int)sizeof(float2);
-    t->xrows = std::max(1, std::min({DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / h, DWHIP_X_LDS_BYTES / xrow}));
+    t->xrows = std::max(1, std::min({DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / std::max(1, h), DWHIP_X_LDS_BYTES / xrow}));
     // a column tile holds B pencils of n complex values in LDS
     t->ysmall = ny * DWHIP_YCOLS_LINE <= DWHIP_YMAXE * DWHIP_YTHR_SMALL;
     const int ylim = std::min(DWHIP_YMAXE * (t->ysmall ? DWHIP_YTHR_SMALL : DWHIP_CTHR),

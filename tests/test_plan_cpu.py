@@ -100,3 +100,18 @@ def test_statistics_cover_the_psf_and_fit_the_spectrum(probe):
         assert 1 <= blocks <= 1024 and 32 * blocks <= room
         n = max(M * N * P, pM * pN * pP)
         assert blocks in (1024, room // 32, max(1, n // 2048))
+
+
+def test_any_size_plan_of_one_column(probe):
+    """A job one voxel wide has a plan on the any-size path too."""
+    body = """
+        DwhipJob j;
+        j.allow_ext = false;
+        dwhip_params p;
+        dwhip_params_default(&p, 2);
+        p.border_quality = 0;
+        const float* im = (const float*)(uintptr_t)256;
+        if (dwhip_job_plan(&j, im, v[0], v[1], v[2], im, 1, 1, 1, &p, nullptr) != DWHIP_OK) return 1;
+        printf("%d\\n", j.generic);
+    """
+    assert probe(body, [(1, 1021, 31), (1, 1, 2503)]) == [[1], [1]]
