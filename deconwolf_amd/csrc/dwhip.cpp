@@ -142,14 +142,39 @@ bool dwhip_fast_size_ok(const int64_t* w)
     return true;
 }
 
+// Whether an extended job of period w transformed at L takes less time per
+// iteration than the any-size path, by what both move (us):
+//   extended   its passes' bytes at the rate their z tiles reach, 2.8 TB/s with
+//              whole lines or half ones (8 columns and more), 1.8 with 4, 1.15
+//              with 2 (z above 1280), and nine launches
+//   any-size   60 ps per voxel, 36 more for each axis that needs Bluestein's form,
+//              and fourteen launches
+// 251 x 249 x 131 (three Bluestein axes, PSF 31 x 31 x 131) takes 427 us extended
+// and 1697 on the any-size path, 375 x 375 x 75 (none, only x odd) 454 and 664;
+// but 125 x 125 x 1500 (none, PSF 125 x 125 x 5) 3200 and 1299, 63 x 61 x 701 with a
+// PSF as long 1027 and 419: where the padding doubles axes that the any-size path
+// transforms at their length, or the z tiles shrink to two columns.  Over 270 sizes
+// (25 to 2011 per axis, PSFs of a few values to the whole period) the path taken is
+// at most 16 % slower than the other; always extended, up to 2.5 times slower.
+static bool ext_pays(const int64_t* w, const int64_t* L)
+{
+    const double row = (double)(L[0] / 2 + 1) * sizeof(float2);
+    const double X = row * w[1] * w[2], C = row * L[1] * w[2], K = row * L[1] * L[2];
+    const double voxels = (double)w[0] * w[1] * w[2];
+    DwhipTiles t;
+    dwhip_tile_config(L, &t);
+    const double rate = t.zcols >= 8 ? 2.8e6 : t.zcols == 4 ? 1.8e6 : t.zcols == 2 ? 1.15e6 : 0.6e6;  // bytes per us
+    const double t_ext = (8 * X + 8 * C + 2 * K + 4 * voxels * sizeof(float)) / rate + 45;
+    int bluestein = 0;
+    for (int d = 0; d < 3; ++d) bluestein += !is_smooth(w[d]);
+    return t_ext <= voxels * 1e-6 * (60 + 36 * bluestein) + 70;
+}
+
 // Transform lengths L of an extended job: a work size w the fused passes
 // cannot transform, its circular convolution of period w[d] computed as one
 // of length L[d] >= w[d] + p[d] - 1 that they can (an axis they transform at
-// w[d] keeps it).  Against the any-size path (Bluestein, a pair of length
-// >= 2 w[d] - 1 transforms per axis, elementwise steps unfused), ten iterations
-// of 1115 x 1115 x 100 with a 181 x 181 x 79 PSF, transformed at 1296 x 1296 x
-// 100, take 36.5 ms instead of 153.7.  False when an axis has no such length or its PSF is
-// longer than the period (the any-size path then runs the job).
+// w[d] keeps it).  False when an axis has no such length, its PSF is longer
+// than the period, or the any-size path is the faster one (it then runs the job).
 bool dwhip_ext_size(const int64_t* w, int64_t pM, int64_t pN, int64_t pP, int64_t* L)
 {
     const int64_t p[3] = {pM, pN, pP};
@@ -162,7 +187,7 @@ bool dwhip_ext_size(const int64_t* w, int64_t pM, int64_t pN, int64_t pP, int64_
             continue;
         }
         const int64_t need = w[d] + p[d] - 1;
-        // the searches below end: every axis plans some length up to its limit
+        // the longest transform of each axis (z plans end before it, at 7^4)
         const int64_t limit = d == 0 ? 2 * DWHIP_XMAXE * DWHIP_XTHR : d == 1 ? DWHIP_YMAXE * DWHIP_CTHR
                                                                              : DWHIP_ZMAXE * DWHIP_ZTHR;
         L[d] = 0;
@@ -175,7 +200,7 @@ bool dwhip_ext_size(const int64_t* w, int64_t pM, int64_t pN, int64_t pP, int64_
         }
         if (L[d] == 0) return false;
     }
-    return dwhip_fast_size_ok(L);
+    return dwhip_fast_size_ok(L) && ext_pays(w, L);
 }
 
 int dwhip_work_size(int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN, int64_t pP,

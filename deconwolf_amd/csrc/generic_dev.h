@@ -1,10 +1,11 @@
 // Device descriptors of the any-size path: deconwolf's SHB and RL loops for
-// work sizes neither the fused passes nor their extended jobs (JobDev.ext)
+// work sizes neither the fused passes nor their extended jobs (dwhip_ext_size)
 // transform: border quality 0 and 1 at deconwolf's exact size, whose extents
 // may hold any prime factor or be odd, where no padded length has a plan, the
-// PSF is longer than the period, or the padded spectra do not fit.  Each axis is a complex FFT of its length n: Stockham passes in LDS
-// with radices 2, 3, 4, 5 and 7 when n factors into them, and Bluestein's
-// chirp-z form otherwise (a length-m FFT pair with m >= 2n - 1 that does
+// PSF is longer than the period, the padded spectra do not fit, or this path
+// is the faster one.  Each axis is a complex FFT of its length n: Stockham
+// passes in LDS with radices 2, 3, 4, 5 and 7 when n factors into them, and
+// Bluestein's chirp-z form otherwise (a length-m FFT pair with m >= 2n - 1 that does
 // factor).  The volumes are real, so x is a real transform of any length:
 // two real rows as the real and imaginary parts of one complex row, their
 // half spectra (nx/2 + 1 bins) separated after the forward transform and

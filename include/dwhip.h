@@ -130,8 +130,9 @@ int dwhip_init(void);
  * 5 and 7 (the image region is unchanged by that padding); for quality 0
  * and 1 the reference size itself, run by the fused passes when it factors
  * that way, else by them at a longer length (the period continued as far as
- * the PSF reaches), else by the any-size path (odd extents and any prime
- * factor, through Bluestein's form; extents up to about 4800).
+ * the PSF reaches) or by the any-size path, whichever takes less time (odd
+ * extents and any prime factor, through Bluestein's form; extents up to about
+ * 4800).
  * Returns DWHIP_OK or DWHIP_ERR_SIZE (an extent beyond both).
  */
 int dwhip_work_size(int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN, int64_t pP,

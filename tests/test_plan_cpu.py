@@ -102,6 +102,40 @@ def test_statistics_cover_the_psf_and_fit_the_spectrum(probe):
         assert blocks in (1024, room // 32, max(1, n // 2048))
 
 
+# image, PSF, bq 0: sizes timed on both paths (us per iteration, extended and
+# any-size) and the one that runs them; near ties in between are left out
+PATHS = [
+    ((61, 61, 31), (61, 61, 31), "ext"),             # 128, 170
+    ((251, 249, 131), (31, 31, 131), "ext"),         # 427, 1697
+    ((375, 375, 75), (375, 375, 75), "ext"),         # 546, 663
+    ((1021, 1021, 31), (1021, 1021, 31), "ext"),     # 2941, 4767
+    ((25, 25, 250), (9, 9, 5), "ext"),               # 83, 102
+    ((61, 61, 1008), (9, 9, 5), "ext"),              # 334, 468
+    ((125, 125, 1500), (125, 125, 5), "any"),        # 3200, 1299
+    ((125, 125, 640), (125, 125, 5), "any"),         # 938, 601
+    ((63, 61, 701), (63, 61, 701), "any"),           # 1027, 419
+    ((63, 61, 1009), (31, 31, 1009), "any"),         # 913, 569
+    ((25, 25, 1800), (9, 9, 5), "any"),              # 235, 204
+    # no choice: a depth no padded plan covers
+    ((5, 5, 2503), (3, 3, 5), "any"),
+]
+
+
+def test_extended_or_any_size_by_time(probe):
+    body = """
+        DwhipJob j;
+        dwhip_params p;
+        dwhip_params_default(&p, 2);
+        p.border_quality = 0;
+        const float* im = (const float*)(uintptr_t)256;
+        if (dwhip_job_plan(&j, im, v[0], v[1], v[2], im, v[3], v[4], v[5], &p, nullptr) != DWHIP_OK) return 1;
+        printf("%d %d\\n", j.ext, j.generic);
+    """
+    got = probe(body, [a + b for a, b, _ in PATHS])
+    for (shape, psf, want), (ext, gen) in zip(PATHS, got):
+        assert (ext, gen) == ((1, 0) if want == "ext" else (0, 1)), (shape, psf)
+
+
 def test_any_size_plan_of_one_column(probe):
     """A job one voxel wide has a plan on the any-size path too."""
     body = """
