@@ -117,6 +117,7 @@ struct Table {
     std::vector<EngJob*> jobs;
     BatchDev* bd() const { return (BatchDev*)dev; }
     JobDev* jd() const { return (JobDev*)(dev + 64); }
+    const JobDev& host_job(int i) const { return ((const JobDev*)(host + 64))[i]; }
     static size_t bytes(int cap) { return 64 + (size_t)cap * sizeof(JobDev); }
 };
 
@@ -134,6 +135,7 @@ struct dwhip_engine {
     std::vector<EngJob*> active;
     std::map<int64_t, EngJob*> done;
     Table tsetup, tweights, tae, tfh, tae2, tfh2;
+    Table tfirst, tfirst2;  // a step's first round, when jobs start in it
     // graph of one full round of the current active set (both groups),
     // replayed for the rounds of a step before its last; its tables stay
     // as captured until the active set changes
@@ -173,7 +175,16 @@ bool dev_stop_job(const EngJob* j)
     return j->prm.iter_type != DWHIP_ITER_FIXED && !dwhip_job_solo(&j->j);
 }
 
-int table_build(Table* t, const std::vector<EngJob*>& jobs, hipStream_t s)
+// In iteration 0 of a flat start only pass E and the adjoint half have work
+bool starts_flat(const EngJob* j)
+{
+    return j->j.d.flat && j->j.host_iter == 0 && !dwhip_job_solo(&j->j);
+}
+
+// forward: the table runs a round's forward passes (A to D), in which a job
+// that starts flat has no tiles (its descriptor could tell a tile so, at the
+// price of a load before every tile's first: z passes of one plane 72 -> 89 us)
+int table_build(Table* t, const std::vector<EngJob*>& jobs, hipStream_t s, bool forward = false)
 {
     if ((int)jobs.size() > t->cap) return DWHIP_ERR_ARG;
     t->jobs = jobs;
@@ -191,6 +202,7 @@ int table_build(Table* t, const std::vector<EngJob*>& jobs, hipStream_t s)
         t->ysmall = t->ysmall && jobs[i]->j.tiles.ysmall;
         jh[i] = jobs[i]->j.d;
         jh[i].dev_stop = dev_stop_job(jobs[i]) ? 1 : 0;
+        if (forward && starts_flat(jobs[i])) jh[i].ntile[KIND_X] = jh[i].ntile[KIND_Y] = jh[i].ntile[KIND_Z] = jh[i].ntile[KIND_YD] = 0;
         for (int k = 0; k < KIND_N; ++k) {
             jh[i].tile0[k] = t->ntile[k];
             t->ntile[k] += jh[i].ntile[k];
@@ -213,7 +225,8 @@ int table_pass(const Table& t, bool xkind, int mode, hipStream_t s)
                          : dwhip_launch_colpass(mode, t.ysmall ? PASS_V_YSMALL : 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
     if (slot >= 0) {
         double by = 0;
-        for (EngJob* j : t.jobs) by += dwhip_pass_bytes(xkind ? 1 : 0, mode, j->j.d, j->j.host_iter);
+        for (int i = 0; i < t.n; ++i)
+            if (t.host_job(i).ntile[kind] > 0) by += dwhip_pass_bytes(xkind ? 1 : 0, mode, t.jobs[i]->j.d, t.jobs[i]->j.host_iter);
         dwhip_prof_end(s, slot, (xkind ? 0 : 7) + mode, by);
     }
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, xkind ? "batched x pass" : "batched column pass", __LINE__);
@@ -377,7 +390,7 @@ int dwhip_engine_create(const dwhip_engine_config* cfg, void* stream, dwhip_engi
     E->arena.init(cfg->hbm_budget);
     const int cap = cfg->max_active;
     if (table_alloc(&E->tsetup, cap) || table_alloc(&E->tweights, cap) || table_alloc(&E->tae, cap) ||
-        table_alloc(&E->tfh, cap) || table_alloc(&E->gae, cap)) {
+        table_alloc(&E->tfh, cap) || table_alloc(&E->gae, cap) || table_alloc(&E->tfirst, cap)) {
         dwhip_engine_destroy(E);
         return DWHIP_ERR_NOMEM;
     }
@@ -387,7 +400,8 @@ int dwhip_engine_create(const dwhip_engine_config* cfg, void* stream, dwhip_engi
         return DWHIP_ERR_HIP;
     }
     if (cfg->groups == 2) {
-        if (table_alloc(&E->tae2, cap) || table_alloc(&E->tfh2, cap) || table_alloc(&E->gae2, cap)) {
+        if (table_alloc(&E->tae2, cap) || table_alloc(&E->tfh2, cap) || table_alloc(&E->gae2, cap) ||
+            table_alloc(&E->tfirst2, cap)) {
             dwhip_engine_destroy(E);
             return DWHIP_ERR_NOMEM;
         }
@@ -422,6 +436,8 @@ void dwhip_engine_destroy(dwhip_engine* E)
     table_free(&E->tfh2);
     table_free(&E->gae);
     table_free(&E->gae2);
+    table_free(&E->tfirst);
+    table_free(&E->tfirst2);
     if (E->graph) (void)hipGraphExecDestroy(E->graph);
     if (E->cs2) (void)hipStreamDestroy(E->cs2);
     if (E->ev_fork) (void)hipEventDestroy(E->ev_fork);
@@ -539,7 +555,7 @@ static int group_round(Table* tae, Table* tfh, const std::vector<EngJob*>& all, 
         if (full) fh.push_back(j);
     }
     if (jobs.empty()) return DWHIP_OK;
-    RCHK(table_build(tae, jobs, s));
+    RCHK(table_build(tae, jobs, s, true));
     RCHK(table_build(tfh, fh, s));
     RCHK(table_pass(*tae, true, XM_UPDATE, s));
     RCHK(table_pass(*tae, false, CM_YFWD, s));
@@ -553,39 +569,46 @@ static int group_round(Table* tae, Table* tfh, const std::vector<EngJob*>& all, 
     return DWHIP_OK;
 }
 
-// The passes of one full round (every job transforms its adjoint half) over
-// table t, which serves as both the A-E and the F-H table.
-static int full_round(const Table& t, hipStream_t s)
+// The passes of one full round (every job transforms its adjoint half):
+// forward half over table t, adjoint half over table u.
+static int full_round(const Table& t, const Table& u, hipStream_t s)
 {
     RCHK(table_pass(t, true, XM_UPDATE, s));
     RCHK(table_pass(t, false, CM_YFWD, s));
     RCHK(table_pass(t, false, CM_ZCONV, s));
     RCHK(table_pass(t, false, CM_YINV_IMG, s));
     RCHK(table_pass(t, true, XM_RATIO, s));
-    RCHK(table_pass(t, false, CM_YFWD_IMG, s));
-    RCHK(table_pass(t, false, CM_ZCONVJ, s));
-    RCHK(table_pass(t, false, CM_YINV, s));
-    ECHK(dwhip_launch_round_end(t.bd(), t.jd(), t.n, 1, s));
+    RCHK(table_pass(u, false, CM_YFWD_IMG, s));
+    RCHK(table_pass(u, false, CM_ZCONVJ, s));
+    RCHK(table_pass(u, false, CM_YINV, s));
+    ECHK(dwhip_launch_round_end(u.bd(), u.jd(), u.n, 1, s));
     return DWHIP_OK;
 }
 
-// Capture body: group 0 on the capture stream, group 1 (if any) on a
-// branch forked from it and joined back.
+// One full round of both groups: group 0 on s, group 1 (if any) on a branch
+// forked from it and joined back.  The adjoint half runs over gae, gae2; the
+// forward half over t, t2.
+static int both_rounds(dwhip_engine* E, const Table& t, const Table& t2, hipStream_t s)
+{
+    const bool two = E->gae2.n > 0;
+    if (two) {
+        ECHK(hipEventRecord(E->ev_fork, s));
+        ECHK(hipStreamWaitEvent(E->cs2, E->ev_fork, 0));
+    }
+    RCHK(full_round(t, E->gae, s));
+    if (two) {
+        RCHK(full_round(t2, E->gae2, E->cs2));
+        ECHK(hipEventRecord(E->ev_join, E->cs2));
+        ECHK(hipStreamWaitEvent(s, E->ev_join, 0));
+    }
+    return DWHIP_OK;
+}
+
+// Capture body
 static int capture_round(void* ctx, hipStream_t cs)
 {
     dwhip_engine* E = (dwhip_engine*)ctx;
-    const bool two = E->gae2.n > 0;
-    if (two) {
-        ECHK(hipEventRecord(E->ev_fork, cs));
-        ECHK(hipStreamWaitEvent(E->cs2, E->ev_fork, 0));
-    }
-    RCHK(full_round(E->gae, cs));
-    if (two) {
-        RCHK(full_round(E->gae2, E->cs2));
-        ECHK(hipEventRecord(E->ev_join, E->cs2));
-        ECHK(hipStreamWaitEvent(cs, E->ev_join, 0));
-    }
-    return DWHIP_OK;
+    return both_rounds(E, E->gae, E->gae2, cs);
 }
 
 // Rounds this step runs: up to the next known completion (the fewest
@@ -605,8 +628,9 @@ static int step_rounds(const dwhip_engine* E)
     return std::max(1, r);
 }
 
-// Replays `n` full rounds of the active groups on E->s from one captured
-// round, capturing it again when the groups changed.
+// `n` full rounds of the active groups on E->s, replayed from one captured
+// round, which is captured again when the groups changed; a round that jobs
+// start in is launched directly, without their forward passes.
 static int graph_rounds(dwhip_engine* E, const std::vector<EngJob*>* grp, int n)
 {
     if (n <= 0) return DWHIP_OK;
@@ -625,8 +649,16 @@ static int graph_rounds(dwhip_engine* E, const std::vector<EngJob*>* grp, int n)
         E->graph_jobs[0] = ids[0];
         E->graph_jobs[1] = ids[1];
     }
-    for (int k = 0; k < n; ++k) ECHK(hipGraphLaunch(E->graph, E->s));
-    E->graph_launches += n;
+    int direct = 0;
+    for (int g = 0; g < 2; ++g)
+        for (const EngJob* j : grp[g]) direct |= starts_flat(j) ? 1 : 0;
+    if (direct) {
+        RCHK(table_build(&E->tfirst, grp[0], E->s, true));
+        if (E->tfirst2.cap) RCHK(table_build(&E->tfirst2, grp[1], E->s, true));
+        RCHK(both_rounds(E, E->tfirst, E->tfirst2, E->s));
+    }
+    for (int k = direct; k < n; ++k) ECHK(hipGraphLaunch(E->graph, E->s));
+    E->graph_launches += n - direct;
     for (int g = 0; g < 2; ++g)
         for (EngJob* j : grp[g]) j->j.host_iter += n;
     E->rounds += n;

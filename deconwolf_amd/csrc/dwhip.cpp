@@ -1319,7 +1319,6 @@ int dwhip_fft3_device(float* vol, float* spec, int64_t nx, int64_t ny, int64_t n
     // point U0 at the caller's volume
     JobDev d2 = d;
     d2.U0 = vol;
-    d2.flat = 0;  // the passes of a loop's iteration 0 would do nothing
     hipError_t e = hipMemcpy(job.jd, &d2, sizeof(d2), hipMemcpyHostToDevice);
     const DwhipTiles& t = job.tiles;
     const size_t rowb = (size_t)d.hc * sizeof(float2), pitch = (size_t)d.hcs * sizeof(float2);

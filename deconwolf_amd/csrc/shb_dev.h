@@ -64,8 +64,9 @@ struct JobDev {
     int bg_auto;
     int start_identity; // start from start_img (or im) inserted, instead of flat
     // 1: flat start.  Iteration 0's forward model of a constant is the constant
-    // times the PSF's sum, so its update, y, z and y-inverse passes do nothing
-    // and its ratio pass starts from that value
+    // times the PSF's sum: its update, y, z and y-inverse passes are not launched
+    // (a batch's table has no tiles of theirs for the job) and its ratio pass
+    // starts from that value
     int flat;
     int niter;          // iterations requested (nIter, or maxiter for REL/ABS)
     int rl;             // 1: Richardson-Lucy (method_rl.c), 0: SHB (method_shb.c)

@@ -390,8 +390,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             if (!any) return;
         }
         const int iter = (MODE == XM_UPDATE || MODE == XM_RATIO) ? st->iter : 0;
-        const bool flat0 = J.flat && iter == 0;
-        if (MODE == XM_UPDATE && flat0) return;
+        const bool flat0 = MODE == XM_RATIO && J.flat && iter == 0;
         const bool inv = (MODE == XM_RATIO && !flat0) || MODE == XM_WEIGHTS || MODE == XM_STORE ||
                          (MODE == XM_UPDATE && iter > 0);
         const bool fwd = MODE != XM_WEIGHTS && MODE != XM_STORE;
@@ -476,10 +475,10 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
         }
 
         // the PSF's sum: the OTF's first value without its scale
-        const float psum = (MODE == XM_UPDATE && J.rl && J.has_w) || (MODE == XM_RATIO && flat0)
+        const float psum = (MODE == XM_UPDATE && J.rl && J.has_w) || flat0
                                ? ldg(gp(J.K)).x * (((float)J.nx * (float)J.ny) * (float)J.nz)
                                : 0.f;
-        if (MODE == XM_RATIO && flat0) {
+        if (flat0) {
             // y = H p of p = x_0 (SHB: not below bg), a constant
             const float p0 = !J.rl && st->c0 < st->bg ? st->bg : st->c0;
             const float y0 = p0 * psum;
@@ -1094,8 +1093,6 @@ void k_colpass(const BatchDev* __restrict__ bd, const JobDev* __restrict__ jobs)
         const int t = (ykind && (int)gridDim.x == total) ? xcd_tile(t0, total) : t0;
         const JobDev& J = jobs[find_job(jobs, njobs, kind, t)];
         if (J.dev_stop && gp(J.st)->stop) continue;  // the stopping rule ended this job
-        if ((MODE == CM_YFWD || MODE == CM_ZCONV || MODE == CM_YINV_IMG) && J.flat && gp(J.st)->iter == 0)
-            continue;  // iteration 0 of a flat start has no transform
         const int lt = t - J.tile0[kind];
         const int hcs = J.hcs, ny = J.ny;
         const int B = ykind ? J.ycols : J.zcols;
