@@ -6,13 +6,12 @@
 // Per-mode build tunables of the two iteration passes: occupancy target
 // (waves per SIMD) and element chunk of the update (XM_UPDATE = 3) and
 // ratio (XM_RATIO = 4) passes, over the x-pass-wide DWHIP_X_WAVES / XCHUNK.
-// Both are held to three waves per SIMD (168 VGPRs; their LDS tiles allow three
-// workgroups per CU): without the bound the compiler takes 170 in some of them.
+// The ratio pass is held to three waves per SIMD (168 VGPRs; its LDS tiles
+// allow three workgroups per CU): without the bound the compiler takes 170.  The
+// update pass takes 164 by itself, and the bound alone costs it: 700 x 700 x 120
+// 380 us with, 360 without; 256 x 256 x 96 53 and 49.
 #if XMODE == 4 && !defined(DWHIP_XR_WAVES) && !defined(DWHIP_X_WAVES)
 #define DWHIP_XR_WAVES 3
-#endif
-#if XMODE == 3 && !defined(DWHIP_XU_WAVES) && !defined(DWHIP_X_WAVES)
-#define DWHIP_XU_WAVES 3
 #endif
 #if XMODE == 3 && defined(DWHIP_XU_WAVES)
 #define DWHIP_X_WAVES DWHIP_XU_WAVES
