@@ -369,9 +369,21 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
     // first exchange's pad of the forward or the inverse plan; three x
     // workgroups share a CU's LDS
     const std::vector<int> xr = pc && !pc->r[0].empty() ? pc->r[0] : dwhip_radices(h, 0);
-    const int xpad = xr.size() > 1 ? std::max(plan_pad(h, xr.front()), plan_pad(h, xr.back())) : 0;
-    const int xrow = std::max(hc, h + xpad) * (int)sizeof(float2);
-    t->xrows = std::max(1, std::min({DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / std::max(1, h), DWHIP_X_LDS_BYTES / xrow}));
+    const int pad = xr.size() > 1 ? std::max(plan_pad(h, xr.front()), plan_pad(h, xr.back())) : 0;
+    auto rows = [&](int padded) {
+        const int r = std::max(1, std::min({DWHIP_XROWS_MAX, DWHIP_XMAXE * DWHIP_XTHR / std::max(1, h),
+                                            DWHIP_X_LDS_BYTES / (std::max(hc, h + padded) * (int)sizeof(float2))}));
+        return pc && pc->xrows > 0 ? std::min(r, pc->xrows) : r;
+    };
+    // the pad's rows per tile, unless all tiles run at once (three per CU) only
+    // without it: 672 x 784 x 18 in 743 tiles of 19 rows takes 62 us (update) and
+    // 46 (ratio), in 830 of 17 rows 83 and 42; in several turns the pad gains (672 x
+    // 672 x 80 212 -> 206 and 131 -> 118, 448 x 343 x 50 60 -> 56 and 45 -> 43)
+    const int64_t nrows = (int64_t)ny * nz, at_once = 3 * DWHIP_CUS;
+    auto tiles = [&](int padded) { return (nrows + rows(padded) - 1) / rows(padded); };
+    t->xpad = pad > 0 && !(tiles(pad) > at_once && tiles(0) <= at_once);
+    t->xrows = rows(t->xpad ? pad : 0);
+    const int xrow = std::max(hc, h + (t->xpad ? pad : 0)) * (int)sizeof(float2);
     // a column tile holds B pencils of n complex values in LDS
     t->ysmall = ny * DWHIP_YCOLS_LINE <= DWHIP_YMAXE * DWHIP_YTHR_SMALL;
     const int ylim = std::min(DWHIP_YMAXE * (t->ysmall ? DWHIP_YTHR_SMALL : DWHIP_CTHR),
@@ -380,7 +392,6 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
     t->ycols = std::max(1, std::min(64, pow2_floor(ylim / ny)));
     t->zcols = std::max(1, std::min(64, pow2_floor(zlim / nz)));
     if (pc) {
-        if (pc->xrows > 0) t->xrows = std::min(t->xrows, pc->xrows);
         if (pc->ycols > 0) t->ycols = std::min(t->ycols, pow2_floor(pc->ycols));
         if (pc->zcols > 0) t->zcols = std::min(t->zcols, pow2_floor(pc->zcols));
     }
@@ -656,6 +667,7 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
         make_plan_pair(d.ny, 1, &d.pyf, &d.pyi, tw, pc ? &pc->r[1] : nullptr) ||
         make_plan_pair(d.nz, 2, &d.pzf, &d.pzi, tw, pc ? &pc->r[2] : nullptr))
         return DWHIP_ERR_SIZE;
+    if (!j->tiles.xpad) d.pxf.pad = d.pxi.pad = 0;
     j->rtw_off = tw.size();
     for (int k = 0; k < d.h; ++k) {
         const double a = -2.0 * M_PI * (double)k / (double)d.nx;

@@ -14,6 +14,7 @@
 
 struct DwhipTiles {
     int xrows, ycols, zcols;
+    bool xpad;    // x plans keep their first exchange's pad (FftPlanDev.pad)
     bool ysmall;  // y tiles fit workgroups of DWHIP_YTHR_SMALL threads
     int ntile[KIND_N];
     size_t lds[KIND_N];

@@ -78,6 +78,7 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #define DWHIP_XROWS_MAX 64  // rows per X tile at most
 #endif
 #define DWHIP_MAX_RADIX 25
+#define DWHIP_CUS 256  // compute units of the GPU
 #define DWHIP_STAT_BLOCKS 1024  // workgroups of the set-up statistics at most
 #ifndef DWHIP_X_STAGE_LDS
 #define DWHIP_X_STAGE_LDS 1  // X passes stage their half-spectrum rows in LDS before the C2R

@@ -149,3 +149,32 @@ def test_any_size_plan_of_one_column(probe):
         printf("%d\\n", j.generic);
     """
     assert probe(body, [(1, 1021, 31), (1, 1, 2503)]) == [[1], [1]]
+
+
+# work sizes: image, x rows per tile, values of the pad (forward, inverse plan)
+PADS = [
+    ((672, 784, 18), 19, 0, 0),      # 743 tiles without the pad, 830 with it
+    ((672, 672, 80), 17, 42, 0),     # several turns either way
+    ((672, 784, 17), 19, 0, 0),      # 702 and 784
+    ((672, 784, 16), 17, 42, 0),     # one turn either way
+    ((256, 256, 96), 46, 8, 16),     # 16 * 8
+    ((1250, 1215, 140), 10, 0, 0),   # 25 * 25: odd
+]
+
+
+def test_x_pad_keeps_tiles_at_once(probe):
+    """The padded exchange of the x rows is given up where its rows would take
+    the tiles from one turn (three workgroups per CU) to two; plan and tiles agree."""
+    body = """
+        DwhipJob j;
+        dwhip_params p;
+        dwhip_params_default(&p, 2);
+        for (int d = 0; d < 3; ++d) p.work[d] = v[d];
+        const float* im = (const float*)(uintptr_t)256;
+        if (dwhip_job_plan(&j, im, v[0] / 2, v[1] / 2, v[2] / 2, im, 1, 1, 1, &p, nullptr) != DWHIP_OK) return 1;
+        printf("%d %d %d %zu\\n", j.tiles.xrows, j.d.pxf.pad, j.d.pxi.pad, j.tiles.lds[KIND_X]);
+    """
+    for (w, rows, fwd, inv), got in zip(PADS, probe(body, [w for w, *_ in PADS])):
+        assert got[:3] == [rows, fwd, inv], w
+        h = w[0] // 2
+        assert got[3] >= rows * 8 * max(h + 1, h + fwd, h + inv)
