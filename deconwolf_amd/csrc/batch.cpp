@@ -222,7 +222,8 @@ int table_pass(const Table& t, bool xkind, int mode, hipStream_t s)
     if (t.n == 0 || t.ntile[kind] == 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
     hipError_t e = xkind ? dwhip_launch_xpass(mode, 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s)
-                         : dwhip_launch_colpass(mode, t.ysmall ? PASS_V_YSMALL : 0, t.bd(), t.jd(), t.ntile[kind], t.lds[kind], s);
+                         : dwhip_launch_colpass(mode, pass_ysmall(t.ysmall, t.ntile[kind]) ? PASS_V_YSMALL : 0, t.bd(), t.jd(),
+                                                t.ntile[kind], t.lds[kind], s);
     if (slot >= 0) {
         double by = 0;
         for (int i = 0; i < t.n; ++i)

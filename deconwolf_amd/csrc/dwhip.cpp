@@ -838,7 +838,7 @@ int dwhip_pass_c(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* 
 {
     if (ntile <= 0) return DWHIP_OK;
     const int slot = dwhip_prof_begin(s);
-    const int variant = (j->ext && bd != j->obd ? PASS_V_EXT : 0) | (j->tiles.ysmall ? PASS_V_YSMALL : 0);
+    const int variant = (j->ext && bd != j->obd ? PASS_V_EXT : 0) | (pass_ysmall(j->tiles.ysmall, ntile) ? PASS_V_YSMALL : 0);
     hipError_t e = dwhip_launch_colpass(mode, variant, bd, jd, ntile, lds, s);
     if (slot >= 0) dwhip_prof_end(s, slot, 7 + mode, dwhip_pass_bytes(0, mode, j->d, 0));
     return e == hipSuccess ? DWHIP_OK : dwhip_hip_fail(e, "column pass", __LINE__);

@@ -42,6 +42,7 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #ifndef DWHIP_XTHR
 #define DWHIP_XTHR 256   // threads per X-pass workgroup
 #endif
+#define DWHIP_CUS 256  // compute units of the GPU
 #ifndef DWHIP_CTHR
 #define DWHIP_CTHR 1024  // threads per workgroup, Y passes (long pencils)
 #endif
@@ -51,8 +52,12 @@ __host__ __device__ constexpr int cmode_kind(int m)
 // with 1024 threads, 79-88 with 512; of 512 x 512 x 64: 42-45, 37-40.  Longer
 // pencils would leave 8 columns, half lines: 1250 x 1215 x 140 takes 383 us with
 // 1024 threads and 16 columns, 522 with 512 and 8.
+// A pass with fewer tiles than CUs leaves no second tile to overlap with and runs
+// the larger workgroups (the tiles stay): y passes of 48 x 100 x 56, one tile per
+// plane, 11-12 us with 512 threads, 10 with 1024.
 #define DWHIP_YTHR_SMALL 512
 #define DWHIP_YCOLS_LINE 16
+inline bool pass_ysmall(bool fits, int ntile) { return fits && ntile >= DWHIP_CUS; }
 #ifndef DWHIP_ZTHR
 #define DWHIP_ZTHR 512   // threads per workgroup, Z passes
 #endif
@@ -78,7 +83,6 @@ __host__ __device__ constexpr int cmode_kind(int m)
 #define DWHIP_XROWS_MAX 64  // rows per X tile at most
 #endif
 #define DWHIP_MAX_RADIX 25
-#define DWHIP_CUS 256  // compute units of the GPU
 #define DWHIP_STAT_BLOCKS 1024  // workgroups of the set-up statistics at most
 #ifndef DWHIP_X_STAGE_LDS
 #define DWHIP_X_STAGE_LDS 1  // X passes stage their half-spectrum rows in LDS before the C2R
