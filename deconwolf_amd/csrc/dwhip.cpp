@@ -410,47 +410,27 @@ void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* p
 
 static size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// At least what dwhip_job_plan lays out for the job, on the any-size path where
+// that is the path that needs least, and at most some KiB more.
 size_t dwhip_job_bytes(const int64_t* work, int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN,
                        int64_t pP, int border_quality, int niter)
 {
-    int64_t L[3];
-    if (!dwhip_fast_size_ok(work) && dwhip_ext_size(work, pM, pN, pP, L)) {
-        // extended job: spectra of the transform's rows and columns (C in the
-        // data's planes, K in all), U0, U1 (and W) of the data
-        const size_t hcs = round_up(L[0] / 2 + 1, 16);
-        const size_t V = round_up(work[0], 2) * work[1] * work[2];
-        DwhipTiles t;
-        dwhip_tile_config(L, &t);
-        size_t b = hcs * L[1] * (work[2] + L[2]) * sizeof(float2) + (border_quality > 0 ? 3 : 2) * V * sizeof(float);
-        b += (size_t)ratio_tiles(work[1], work[2], t.xrows) * sizeof(double);
-        b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-        b += 4096 + 2 * sizeof(JobDev);
-        for (int d = 0; d < 3; ++d) b += 3 * (size_t)L[d] * sizeof(float2);
-        return b;
-    }
-    if (!dwhip_fast_size_ok(work)) {
-        // any-size path: half spectra Z and K, U0, U1 (and W), partials, tables
-        const size_t V = (size_t)work[0] * work[1] * work[2];
-        const size_t Vh = round_up(work[0] / 2 + 1, 16) * work[1] * work[2];
-        size_t b = 2 * Vh * sizeof(float2) + (border_quality > 0 ? 3 : 2) * V * sizeof(float);
-        b += (size_t)dwhip_generic_ratio_grid() * sizeof(double);
-        b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-        b += 4096 + sizeof(GenDev) + sizeof(JobDev);
-        for (int d = 0; d < 3; ++d) b += 8 * (size_t)work[d] * sizeof(float2);  // twiddles, chirps, filters
-        return b;
-    }
-    const size_t h = work[0] / 2, hcs = round_up(h + 1, 16);
+    (void)M; (void)pM; (void)pN; (void)pP;
     const size_t V = (size_t)work[0] * work[1] * work[2];
-    const size_t Vc = hcs * work[1] * work[2];
-    DwhipTiles t;
-    dwhip_tile_config(work, &t);
-    size_t b = 2 * Vc * sizeof(float2);                  // C, K
+    const size_t Vc = round_up(work[0] / 2 + 1, 16) * work[1] * work[2];
+    size_t b = 2 * Vc * sizeof(float2);                    // C, K
     b += (border_quality > 0 ? 3 : 2) * V * sizeof(float); // U0, U1, W
-    b += (size_t)std::max(t.ntile[KIND_X], ratio_tiles(N, P, t.xrows)) * sizeof(double);
-    b += (size_t)(niter + 1) * (sizeof(float) + sizeof(double));
-    b += 4096;
-    (void)M;
-    return b;
+    b += (size_t)std::max(1, niter) * (sizeof(float) + sizeof(double));
+    b += 64 + 2 * sizeof(JobDev) + sizeof(GenDev) + sizeof(JobState);
+    b += 12 * 256;  // every buffer starts on 256 bytes
+    if (!dwhip_fast_size_ok(work))
+        return b + (size_t)dwhip_generic_ratio_grid() * sizeof(double) + dwhip_generic_table_bytes(work);
+    // twiddles of both directions and of the rows' split, the partial sums
+    DwhipPlanChoice pc;
+    DwhipTiles t;
+    dwhip_tile_config(work, &t, dwhip_plan_cached(work, &pc) ? &pc : nullptr);
+    b += (3 * (size_t)(work[0] / 2) + 2 * (size_t)(work[1] + work[2])) * sizeof(float2);
+    return b + (size_t)std::max(t.ntile[KIND_X], ratio_tiles(N, P, t.xrows)) * sizeof(double);
 }
 
 // ---------------------------------------------------------------------------

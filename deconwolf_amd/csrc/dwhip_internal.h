@@ -133,3 +133,4 @@ int dwhip_generic_setup(const DwhipJob* j, hipStream_t s);
 int dwhip_generic_round(DwhipJob* j, bool full, hipStream_t s);
 int dwhip_generic_final_update(DwhipJob* j, hipStream_t s);
 int dwhip_generic_ratio_grid();
+size_t dwhip_generic_table_bytes(const int64_t* w);

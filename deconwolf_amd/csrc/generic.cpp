@@ -209,6 +209,18 @@ size_t dwhip_generic_lds(const DwhipJob* j, int axis)
 
 int dwhip_generic_ratio_grid() { return kRatioGrid; }
 
+// bytes of a job's twiddle and Bluestein tables (dwhip_generic_plan)
+size_t dwhip_generic_table_bytes(const int64_t* w)
+{
+    size_t n = 0;
+    for (int d = 0; d < 3; ++d) {
+        bool blue = false;
+        const size_t m = (size_t)gen_fft_len((int)w[d], &blue);
+        n += m + (blue ? (size_t)w[d] + 2 * m : 0);
+    }
+    return n * sizeof(float2);
+}
+
 // Points the GenDev at the job's buffers (after dwhip_job_bind has laid
 // them out) and queues its upload.
 int dwhip_generic_bind(DwhipJob* j, char* gdev, hipStream_t s)

@@ -160,7 +160,10 @@ int dwhip_plan_tune(const int64_t *work, int retune, double *tuned_ms, double *r
 int dwhip_plan_cache_path(const char *path);
 int dwhip_plan_get(const int64_t *work, int *radices, int *tiles);
 
-/* Device bytes one job of these sizes needs. */
+/* Device bytes one job of these sizes needs.  A job of border quality 0 or 1
+ * that runs the fused passes at a longer length takes more where there is room
+ * (the static block, an engine's budget, device memory) and runs in these where
+ * there is not. */
 size_t dwhip_job_bytes(const int64_t *work, int64_t M, int64_t N, int64_t P, int64_t pM,
                        int64_t pN, int64_t pP, int border_quality, int niter);
 

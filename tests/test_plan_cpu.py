@@ -178,3 +178,41 @@ def test_x_pad_keeps_tiles_at_once(probe):
         assert got[:3] == [rows, fwd, inv], w
         h = w[0] // 2
         assert got[3] >= rows * 8 * max(h + 1, h + fwd, h + inv)
+
+
+# image, PSF, bq, iterations: plain, extended and any-size jobs
+BYTES = [(1024, 1024, 60, 181, 181, 79, 2, 50), (128, 128, 32, 127, 127, 63, 2, 1), (701, 512, 211, 31, 9, 1, 2, 10),
+         (40, 36, 16, 9, 9, 7, 2, 250), (1, 1, 1, 1, 1, 1, 2, 1), (2048, 2048, 1, 63, 63, 1, 2, 5),
+         (64, 64, 60, 9, 9, 7, 0, 5), (257, 211, 151, 111, 111, 111, 0, 2), (1024, 1024, 60, 181, 181, 79, 1, 10),
+         (37, 23, 11, 37, 23, 11, 0, 4), (1, 1021, 31, 1, 1, 5, 0, 1), (5, 8, 2503, 3, 3, 5, 0, 3),
+         (2011, 11, 7, 101, 11, 7, 1, 100), (125, 125, 1500, 125, 125, 5, 0, 3)]
+
+
+def test_job_bytes_is_what_a_job_needs(probe):
+    """dwhip_job_bytes covers what a job lays out and asks for little more; a job
+    that also has a larger, extended layout runs in it (the static block, an
+    engine's budget and a failed allocation plan it without the extension)."""
+    body = """
+        dwhip_params p;
+        dwhip_params_default(&p, (int)v[7]);
+        p.border_quality = v[6];
+        int64_t w[3], r[3];
+        if (dwhip_work_size(v[0], v[1], v[2], v[3], v[4], v[5], v[6], w, r) != DWHIP_OK) return 1;
+        size_t most = 0, ext = 0;
+        for (int k = 0; k < 4; ++k) {
+            p.method = k & 1 ? DWHIP_METHOD_RL : DWHIP_METHOD_SHB;
+            DwhipJob j;
+            j.allow_ext = k >= 2;
+            const float* im = (const float*)(uintptr_t)256;
+            if (dwhip_job_plan(&j, im, v[0], v[1], v[2], im, v[3], v[4], v[5], &p, nullptr) != DWHIP_OK) return 1;
+            size_t& n = j.ext ? ext : most;
+            if (j.bytes > n) n = j.bytes;
+        }
+        printf("%zu %zu %zu\\n", dwhip_job_bytes(w, v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]), most, ext);
+    """
+    for job, (est, need, ext) in zip(BYTES, probe(body, BYTES)):
+        assert need <= est <= need + 24 * 1024, job
+        assert not ext or ext > need, job
+    # runs in the static block by its any-size layout
+    est, _, ext = probe(body, [(257, 211, 151, 111, 111, 111, 0, 2)])[0]
+    assert est <= 256 << 20 < ext
