@@ -791,7 +791,11 @@ double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
         // (and W), writes x_k
         if (iter == 0) return (d.rl ? 1 : 2) * V + Xc;
         return 2 * Xc + ((d.rl ? 2 : 3) + (d.has_w ? 1 : 0)) * V;
-    case XM_RATIO: return d.prune ? 2 * imgrows + img : imgrows + Xc + img;
+    case XM_RATIO: {
+        // (iteration 0 of a flat start reads no spectrum)
+        const double in = d.flat && iter == 0 ? 0 : imgrows;
+        return in + (d.prune ? imgrows : Xc) + img;
+    }
     case XM_LOAD: return Vc + V;
     case XM_STORE: return Vc + V;
     default: return 0;
@@ -800,7 +804,7 @@ double dwhip_pass_bytes(int xkind, int mode, const JobDev& d, int iter)
 
 static double host_iter(const DwhipJob* j, int mode)
 {
-    return mode == XM_UPDATE ? (double)j->host_iter : 0;
+    return mode == XM_UPDATE || mode == XM_RATIO ? (double)j->host_iter : 0;
 }
 
 int dwhip_pass_x(int mode, const DwhipJob* j, const BatchDev* bd, const JobDev* jd, int ntile, size_t lds,
