@@ -216,3 +216,27 @@ def test_job_bytes_is_what_a_job_needs(probe):
     # runs in the static block by its any-size layout
     est, _, ext = probe(body, [(257, 211, 151, 111, 111, 111, 0, 2)])[0]
     assert est <= 256 << 20 < ext
+
+
+def test_paths_of_the_gpu_tests(probe):
+    """The sizes that test_gpu_anysize and test_gpu_extended compare with the
+    oracle run extended, those of test_gpu_paths on both paths (the any-size path's
+    own tests take the extension's room away)."""
+    pytest.importorskip("torch")
+    import test_gpu_anysize
+    import test_gpu_extended
+    import test_gpu_paths
+    body = """
+        DwhipJob j;
+        dwhip_params p;
+        dwhip_params_default(&p, 2);
+        p.border_quality = v[6];
+        const float* im = (const float*)(uintptr_t)256;
+        if (dwhip_job_plan(&j, im, v[2], v[1], v[0], im, v[5], v[4], v[3], &p, nullptr) != DWHIP_OK) return 1;
+        printf("%d\\n", j.ext);
+    """
+    cases = [c[0] + c[1] + (c[2],) for c in test_gpu_anysize.CASES]
+    cases += [c[0] + c[1] + (c[3],) for c in test_gpu_extended.CASES]
+    assert probe(body, cases) == [[1]] * len(cases)
+    cases = [c[0] + c[1] + (c[3],) for c in test_gpu_paths.CASES]
+    assert probe(body, cases) == [[1], [0], [0], [0], [0], [1]]
