@@ -53,10 +53,11 @@ __device__ __forceinline__ double shb_alpha(int iter, float alphamax)
 // Richardson-Lucy step x~ (f W) (method_rl.c:85-97) of a pruned job: x~ lacks
 // the adjoint of the ratio's 1e-6 outside the image, 1e-6 (S - P1) with S the
 // PSF's sum and P1 = 1/W; times f W that is 1e-6 f (S W - 1).  W = 0 (P1 below
-// method_rl.c's limit) gives 0 either way.
+// method_rl.c's limit) gives 0 either way, NaN where x~ or f is not finite.
 __device__ __forceinline__ float rl_step(float xt, float f, float w, float psum)
 {
-    return w > 0.f ? fmaf(1e-6f * f, fmaf(psum, w, -1.f), xt * (f * w)) : 0.f;
+    const float x = xt * (f * w);
+    return w > 0.f ? fmaf(1e-6f * f, fmaf(psum, w, -1.f), x) : x;
 }
 
 // p = x + alpha*(x - xp), then p = max(p, bg)  (method_shb.c:333-339):
