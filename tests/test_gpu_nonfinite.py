@@ -23,3 +23,25 @@ def test_nan_reaches_the_whole_volume(method, shape, bq):
     out = (dw.deconvolve_rl_hip if method == dw.METHOD_RL else dw.deconvolve_shb_hip)(im, k, s)
     assert np.isnan(out).all()
     assert np.isnan(got[-1]).all()
+
+
+@pytest.mark.parametrize("method", [dw.METHOD_RL, dw.METHOD_SHB])
+@pytest.mark.parametrize("where", ["image", "psf"])
+def test_infinite_start_has_no_forward_model(method, where):
+    """With an infinite value in the image (the flat start is infinite) or in the
+    PSF, iteration 0's forward model is NaN, which the I-divergence does not count
+    and the squared error hands on (getError, dw.c:1436-1524)."""
+    print("infinite", where, method, flush=True)
+    im, k = _image((12, 20, 24)), _psf((5, 7, 9), (2, 3, 4))
+    if where == "image":
+        im[3, 4, 5] = np.inf
+    else:
+        k[1, 2, 3] = np.inf
+    run = dw.deconvolve_rl_hip if method == dw.METHOD_RL else dw.deconvolve_shb_hip
+    for metric in (dw.METRIC_IDIV, dw.METRIC_MSE):
+        s = dw.DwOpts(nIter=2, iter_type=dw.ITER_FIXED, method=method, metric=metric)
+        run(im, k, s)
+        if metric == dw.METRIC_IDIV:
+            assert s.err_trace[0] == 0
+        else:
+            assert np.isnan(s.err_trace[0])
