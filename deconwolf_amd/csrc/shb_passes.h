@@ -483,7 +483,7 @@ __device__ __forceinline__ void xpass_tile(const JobDev& J, int t, int tid, floa
             // y = H p of p = x_0 (SHB: not below bg), a constant; NaN, as the
             // transforms give, when either factor is not finite
             const float p0 = !J.rl && st->c0 < st->bg ? st->bg : st->c0;
-            const float y0 = p0 * psum + ((p0 - p0) + (psum - psum));
+            const float y0 = isfinite(p0) && isfinite(psum) ? p0 * psum : NAN;
             for (int w = tid; w < nrows * h; w += XTHR) lds[w] = make_float2(y0, y0);
             __syncthreads();
         }

@@ -45,3 +45,25 @@ def test_infinite_start_has_no_forward_model(method, where):
             assert s.err_trace[0] == 0
         else:
             assert np.isnan(s.err_trace[0])
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-3, 1e-6, 1e6])
+@pytest.mark.parametrize("method", [dw.METHOD_RL, dw.METHOD_SHB])
+def test_flat_model_scales_with_the_image(scale, method):
+    """Iteration 0's forward model of a flat start, the start times the PSF's sum,
+    to float32's rounding (2^-23 of it, twice) at every scale of the image."""
+    print("flat model at scale", scale, method, flush=True)
+    im = np.full((12, 3, 40), 3.0 * scale, np.float32)
+    im[::2] *= 0.5
+    k = np.ones((3, 2, 3), np.float32)
+    k[1, 1, 1] = 5
+    k /= k.sum()
+    s = dw.DwOpts(nIter=1, iter_type=dw.ITER_FIXED, borderQuality=1, metric=dw.METRIC_MSE, method=method,
+                  bg_auto=0, bg=0.0)
+    (dw.deconvolve_rl_hip if method == dw.METHOD_RL else dw.deconvolve_shb_hip)(im, k, s)
+    n = np.prod([float(v) for v in s.stats["ref_work"]])
+    y = im.astype(np.float64).sum() / n * k.astype(np.float64).sum()
+    d = im.astype(np.float64) - y
+    # the start, the sum and their product are rounded to float32, the error too
+    tol = 2 * np.abs(d).mean() * y * 4 * 2.0 ** -24 + (d ** 2).mean() * 2.0 ** -24
+    assert abs(float(s.err_trace[0]) - (d ** 2).mean()) <= tol
