@@ -23,7 +23,8 @@ LIB = os.path.join(HERE, "libdwhip.so")
 
 N_XMODES = 7
 N_CMODES = 10
-# modes compiled for extended jobs too (xmode_has_ext, cmode_has_ext)
+# modes compiled for extended jobs too: what such a job runs after its OTF's
+# set-up (k_misc.hip declares their launchers)
 EXT_XMODES = (1, 2, 3, 4)
 EXT_CMODES = (0, 1, 3, 4, 7, 8)
 # y modes, compiled for the small workgroups too

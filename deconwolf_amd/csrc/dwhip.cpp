@@ -559,7 +559,6 @@ int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64
     d.ux = j->ext ? (int)round_up(w[0], 2) : (int)w[0];
     d.uy = (int)w[1];
     d.uz = (int)w[2];
-    d.ext = j->ext ? 1 : 0;
     d.h = d.nx / 2;
     d.hc = d.h + 1;
     d.hcs = (int)round_up(d.hc, 16);  // rows start on 128-byte lines
@@ -719,7 +718,6 @@ int dwhip_job_bind(DwhipJob* j, void* mem, hipStream_t s)
         j->odcopy = d;
         JobDev& o = j->odcopy;
         o.C = o.K;
-        o.ext = 0;
         const int kinds[3] = {KIND_X, KIND_Y, KIND_Z};
         for (int k = 0; k < 3; ++k) j->obh.ntile[kinds[k]] = o.ntile[kinds[k]] = j->otf_tiles[k];
         HIPCHK(hipMemcpyAsync(j->obd, &j->obh, sizeof(j->obh), hipMemcpyHostToDevice, s));

@@ -40,13 +40,11 @@ struct JobDev {
     // transform (work) size; h = nx/2, hc = h+1 complex per x-row, hcs = row stride
     int nx, ny, nz, h, hc, hcs;
     // the real volumes U0, U1 and W: ux x uy x uz values, of which dx along x
-    // hold data (ux = dx rounded up to even in an extended job, else ux = dx =
-    // nx, uy = ny, uz = nz)
+    // hold data.  In an extended job, which the EXT kernels run, the convolution
+    // has period dx, uy, uz but is transformed at nx, ny, nz, the data of every axis
+    // that is longer in the transform continued periodically as far as the PSF
+    // reaches; ux is dx rounded up to even.  Else ux = dx = nx, uy = ny, uz = nz
     int dx, ux, uy, uz;
-    // 1: extended job (the EXT kernels): the convolution has period dx, uy, uz
-    // but is transformed at nx, ny, nz, the data of every axis that is longer
-    // in the transform continued periodically as far as the PSF reaches
-    int ext;
     // image and PSF sizes
     int M, N, P;
     int pM, pN, pP;

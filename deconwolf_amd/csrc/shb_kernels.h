@@ -16,16 +16,6 @@ enum { XM_PSF = 0, XM_ONES = 1, XM_WEIGHTS = 2, XM_UPDATE = 3, XM_RATIO = 4, XM_
 enum { CM_YFWD = 0, CM_YINV = 1, CM_ZOTF = 2, CM_ZCONV = 3, CM_ZCONVJ = 4, CM_ZFWD = 5, CM_ZINV = 6,
        CM_YINV_IMG = 7, CM_YFWD_IMG = 8, CM_YFWD_PSF = 9 };
 #define DWHIP_N_CMODES 10
-// Passes an extended job runs (JobDev.ext): its OTF is set up by the plain
-// passes at the transform size.
-__host__ __device__ constexpr bool xmode_has_ext(int m)
-{
-    return m == XM_ONES || m == XM_WEIGHTS || m == XM_UPDATE || m == XM_RATIO;
-}
-__host__ __device__ constexpr bool cmode_has_ext(int m)
-{
-    return m == CM_YFWD || m == CM_YINV || m == CM_ZCONV || m == CM_ZCONVJ || m == CM_YINV_IMG || m == CM_YFWD_IMG;
-}
 __host__ __device__ constexpr bool cmode_is_y(int m)
 {
     return m == CM_YFWD || m == CM_YINV || m == CM_YINV_IMG || m == CM_YFWD_IMG || m == CM_YFWD_PSF;
