@@ -330,7 +330,9 @@ bool dwhip_plan_cached(const int64_t* w, DwhipPlanChoice* pc)
 int dwhip_plan_ensure(const int64_t* w, int method)
 {
     (void)method;
-    if (!dwhip_fast_size_ok(w)) return DWHIP_OK;  // the any-size path has one plan
+    // the any-size path has one plan; an extended job takes what is cached for its
+    // transform length, else the rule's plan
+    if (!dwhip_fast_size_ok(w)) return DWHIP_OK;
     DwhipPlanChoice c;
     if (dwhip_plan_cached(w, &c)) return DWHIP_OK;
     const int rc = dwhip_plan_tune(w, 0, nullptr, nullptr);

@@ -95,7 +95,8 @@ typedef struct {
  * (FFTW_ESTIMATE / FFTW_MEASURE, src/dw.c:400,1068): RULE plans by rule
  * (and uses a plan measured before, from the plan cache); MEASURE also
  * measures the plans of a new transform size on its first use
- * (dwhip_plan_tune) and caches the result. */
+ * (dwhip_plan_tune) and caches the result; for jobs that run the fused passes
+ * at a longer length than theirs it measures nothing. */
 #define DWHIP_PLAN_RULE 0
 #define DWHIP_PLAN_MEASURE 1
 
@@ -154,7 +155,9 @@ int dwhip_work_size(int64_t M, int64_t N, int64_t P, int64_t pM, int64_t pN, int
  * radices[12] (x-row, y and z forward radices, 4 each, 0-padded) and
  * tiles[3] (x rows, y and z columns per workgroup); returns 1 for a
  * measured plan, 0 for the rule's, or an error.  Sizes the fused passes
- * cannot run give DWHIP_ERR_SIZE (the any-size path has one plan).
+ * cannot run give DWHIP_ERR_SIZE: the any-size path has one plan, and a job
+ * that runs them at a longer length takes a plan cached for that length, else
+ * the rule's.
  */
 int dwhip_plan_tune(const int64_t *work, int retune, double *tuned_ms, double *rule_ms);
 int dwhip_plan_cache_path(const char *path);
@@ -380,10 +383,10 @@ int dwhip_tiles_blend_device(const dwhip_tile *tiles, const float *const *outs, 
  * Kernel timing for measurement.  While enabled, every pass launch is
  * bracketed by HIP events on the stream it runs on and its algorithmic
  * bytes (each operand read or written once) are added up per kernel.
- * dwhip_profile_enable(1) clears the totals.  Kernel ids 0..15 name the
+ * dwhip_profile_enable(1) clears the totals.  Kernel ids 0..16 name the
  * X-pass modes (x_psf, x_ones, x_weights, x_update, x_ratio, x_load,
  * x_store) and column modes (y_fwd, y_inv, z_otf, z_conv, z_convj, z_fwd,
- * z_inv, y_inv_img, y_fwd_img).  No counterpart in deconwolf (its timing is the --times flag,
+ * z_inv, y_inv_img, y_fwd_img, y_fwd_psf).  No counterpart in deconwolf (its timing is the --times flag,
  * src/dw.c:2233-2319).
  */
 int dwhip_profile_enable(int on);
