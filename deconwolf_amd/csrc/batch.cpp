@@ -469,7 +469,8 @@ int dwhip_engine_submit(dwhip_engine* E, const float* im, int64_t M, int64_t N, 
         if (dwhip_work_size(M, N, P, pM, pN, pP, prm->border_quality, w, ref) == DWHIP_OK) {
             for (int d = 0; d < 3; ++d)
                 if (prm->work[d] > 0) w[d] = prm->work[d];
-            const int trc = dwhip_plan_ensure(w, prm->method);
+            const int64_t im_size[3] = {M, N, P};
+            const int trc = dwhip_plan_ensure(w, im_size);
             if (trc != DWHIP_OK) return trc;
         }
     }

@@ -1045,7 +1045,8 @@ static int run_job(const float* im, int64_t M, int64_t N, int64_t P, const float
         if (dwhip_work_size(M, N, P, pM, pN, pP, prm->border_quality, w, ref) == DWHIP_OK) {
             for (int d = 0; d < 3; ++d)
                 if (prm->work[d] > 0) w[d] = prm->work[d];
-            rc = dwhip_plan_ensure(w, prm->method);
+            const int64_t im_size[3] = {M, N, P};
+            rc = dwhip_plan_ensure(w, im_size);
             if (rc != DWHIP_OK) return rc;
         }
     }

@@ -91,8 +91,8 @@ std::vector<int> dwhip_radices(int n, int axis);
 void dwhip_tile_config(const int64_t* w, DwhipTiles* t, const DwhipPlanChoice* pc = nullptr);
 // plan cache and measured planning (tune.cpp)
 bool dwhip_plan_cached(const int64_t* w, DwhipPlanChoice* pc);
-int dwhip_plan_ensure(const int64_t* w, int method);
-extern "C" void dwhip_plan_trial_block(const int64_t* w, size_t* job, size_t* image);
+int dwhip_plan_ensure(const int64_t* w, const int64_t* im);
+extern "C" void dwhip_plan_trial_block(const int64_t* w, const int64_t* im, size_t* job, size_t* image);
 int dwhip_radix_candidates(int n, int axis, std::vector<std::vector<int>>* out);
 int dwhip_job_plan(DwhipJob* j, const float* im_dev, int64_t M, int64_t N, int64_t P, const float* psf_dev,
                    int64_t pM, int64_t pN, int64_t pP, const dwhip_params* prm, const float* start_dev);

@@ -163,16 +163,19 @@ void save_locked()
         if (e_ != hipSuccess) return dwhip_hip_fail(e_, #call, __LINE__); \
     } while (0)
 
-// The image a trial of size w deconvolves: half the transform along each axis.
-void trial_image(const int64_t* w, int64_t* m)
+// The image a trial of size w deconvolves: the job's (im), whose rows are the
+// ratio pass's work, else half the transform along each axis.  On half of a 2048 x
+// 2048 x 1 image (transform 2160 x 2160 x 1) tiles of two rows win, which take the
+// job 316 us per iteration where five take 300.
+void trial_image(const int64_t* w, const int64_t* im, int64_t* m)
 {
-    for (int d = 0; d < 3; ++d) m[d] = std::max<int64_t>(1, w[d] / 2);
+    for (int d = 0; d < 3; ++d) m[d] = im ? im[d] : std::max<int64_t>(1, w[d] / 2);
 }
 
 // Mean time (ms) of the passes of `axis` for plan c on the block mem: cap bytes
 // for the job, then its image.
-int time_axis(const Key& w, int method, const DwhipPlanChoice& c, int axis, void* mem, size_t cap, hipStream_t s,
-              hipEvent_t e0, hipEvent_t e1, double* ms)
+int time_axis(const Key& w, const int64_t* image, int method, const DwhipPlanChoice& c, int axis, void* mem,
+              size_t cap, hipStream_t s, hipEvent_t e0, hipEvent_t e1, double* ms)
 {
     *ms = 1e30;
     DwhipJob j;
@@ -185,7 +188,7 @@ int time_axis(const Key& w, int method, const DwhipPlanChoice& c, int axis, void
     // pass overwrites C); no timed pass reads the PSF
     const float* im = reinterpret_cast<const float*>((const char*)mem + cap);
     int64_t m[3];
-    trial_image(w.data(), m);
+    trial_image(w.data(), image, m);
     int rc = dwhip_job_plan(&j, im, m[0], m[1], m[2], im, 1, 1, 1, &prm, nullptr);
     if (rc != DWHIP_OK) return rc;
     if (j.bytes > cap) return DWHIP_ERR_NOMEM;
@@ -228,7 +231,7 @@ int time_axis(const Key& w, int method, const DwhipPlanChoice& c, int axis, void
 
 // Measures the plans of size w; *tuned / *rule: the summed pass times of
 // the chosen and of the rule's plan.
-int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, double* rule)
+int tune_size(const Key& w, const int64_t* im, int method, DwhipPlanChoice* best, double* tuned, double* rule)
 {
     const int len[3] = {(int)(w[0] / 2), (int)w[1], (int)w[2]};
     std::vector<std::vector<int>> rad[3];
@@ -241,7 +244,7 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
 
     // one block for every candidate
     size_t cap = 0, image = 0;
-    dwhip_plan_trial_block(wv, &cap, &image);
+    dwhip_plan_trial_block(wv, im, &cap, &image);
     void* mem = nullptr;
     TCHK(hipMalloc(&mem, cap + image));
     hipStream_t s = nullptr;
@@ -258,7 +261,7 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
     double sum_best = 0, sum_rule = 0;
     for (int a = 0; a < 3 && rc == DWHIP_OK; ++a) {
         double t_rule = 0;
-        rc = time_axis(w, method, cur, a, mem, cap, s, e0, e1, &t_rule);
+        rc = time_axis(w, im, method, cur, a, mem, cap, s, e0, e1, &t_rule);
         if (rc != DWHIP_OK) break;
         double t_best = t_rule;
         DwhipPlanChoice pick = cur;
@@ -267,7 +270,7 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
             DwhipPlanChoice c = cur;
             c.r[a] = rad[a][i];
             double t = 0;
-            rc = time_axis(w, method, c, a, mem, cap, s, e0, e1, &t);
+            rc = time_axis(w, im, method, c, a, mem, cap, s, e0, e1, &t);
             if (rc == DWHIP_OK && t < t_best * kGain) {
                 t_best = t;
                 pick = c;
@@ -278,7 +281,7 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
             DwhipPlanChoice c = pick;
             (a == 0 ? c.xrows : a == 1 ? c.ycols : c.zcols) = rule_tile[a] / div;
             double t = 0;
-            rc = time_axis(w, method, c, a, mem, cap, s, e0, e1, &t);
+            rc = time_axis(w, im, method, c, a, mem, cap, s, e0, e1, &t);
             if (rc == DWHIP_OK && t < t_best * kGain) {
                 t_best = t;
                 pick = c;
@@ -304,10 +307,10 @@ int tune_size(const Key& w, int method, DwhipPlanChoice* best, double* tuned, do
 
 // Bytes of a trial's block: the job's (the layout depends on the plan only
 // through the twiddle table and the partial sums), then its image's.
-extern "C" void dwhip_plan_trial_block(const int64_t* w, size_t* job, size_t* image)
+extern "C" void dwhip_plan_trial_block(const int64_t* w, const int64_t* im, size_t* job, size_t* image)
 {
     int64_t m[3];
-    trial_image(w, m);
+    trial_image(w, im, m);
     *job = (dwhip_job_bytes(w, m[0], m[1], m[2], 1, 1, 1, 2, 2) + ((size_t)4 << 20) + 255) / 256 * 256;
     *image = (size_t)m[0] * m[1] * m[2] * sizeof(float);
 }
@@ -322,30 +325,7 @@ bool dwhip_plan_cached(const int64_t* w, DwhipPlanChoice* pc)
     return true;
 }
 
-// Tunes w unless a plan for it is cached (used by entry points whose
-// params ask for DWHIP_PLAN_MEASURE).  Measuring only chooses among plans
-// that all run: when it cannot run (no memory for its trial block beside
-// the caller's, a size with nothing to choose), the rule's plan is cached
-// for the size and the job goes on with it.
-int dwhip_plan_ensure(const int64_t* w, int method)
-{
-    (void)method;
-    // the any-size path has one plan; an extended job takes what is cached for its
-    // transform length, else the rule's plan
-    if (!dwhip_fast_size_ok(w)) return DWHIP_OK;
-    DwhipPlanChoice c;
-    if (dwhip_plan_cached(w, &c)) return DWHIP_OK;
-    const int rc = dwhip_plan_tune(w, 0, nullptr, nullptr);
-    if (rc != DWHIP_OK) {
-        (void)hipGetLastError();  // a failed trial allocation leaves its error behind
-        std::lock_guard<std::mutex> lock(g_cache.mu);
-        load_locked();
-        g_cache.plans[Key{w[0], w[1], w[2]}] = DwhipPlanChoice();
-    }
-    return DWHIP_OK;
-}
-
-extern "C" int dwhip_plan_tune(const int64_t* work, int retune, double* tuned_ms, double* rule_ms)
+static int plan_tune(const int64_t* work, const int64_t* im, int retune, double* tuned_ms, double* rule_ms)
 {
     if (!work || work[0] < 2 || work[1] < 1 || work[2] < 1) return DWHIP_ERR_ARG;
     if (!dwhip_fast_size_ok(work)) return DWHIP_ERR_SIZE;
@@ -359,7 +339,7 @@ extern "C" int dwhip_plan_tune(const int64_t* work, int retune, double* tuned_ms
     DwhipPlanChoice best;
     double tb = 0, tr = 0;
     // SHB's passes; RL transforms the same sizes with the same kernels
-    rc = tune_size(k, DWHIP_METHOD_SHB, &best, &tb, &tr);
+    rc = tune_size(k, im, DWHIP_METHOD_SHB, &best, &tb, &tr);
     if (rc != DWHIP_OK) return rc;
     if (tuned_ms) *tuned_ms = tb;
     if (rule_ms) *rule_ms = tr;
@@ -368,6 +348,36 @@ extern "C" int dwhip_plan_tune(const int64_t* work, int retune, double* tuned_ms
     g_cache.plans[k] = best;
     save_locked();
     return DWHIP_OK;
+}
+
+// Tunes w unless a plan for it is cached (used by entry points whose
+// params ask for DWHIP_PLAN_MEASURE).  Measuring only chooses among plans
+// that all run: when it cannot run (no memory for its trial block beside
+// the caller's, a size with nothing to choose), the rule's plan is cached
+// for the size and the job goes on with it.  im: the job's image, which the
+// trials deconvolve.
+int dwhip_plan_ensure(const int64_t* w, const int64_t* im)
+{
+    // the any-size path has one plan; an extended job takes what is cached for its
+    // transform length, else the rule's plan
+    if (!dwhip_fast_size_ok(w)) return DWHIP_OK;
+    for (int d = 0; d < 3; ++d)
+        if (im[d] > w[d]) return DWHIP_OK;  // the job is refused for it
+    DwhipPlanChoice c;
+    if (dwhip_plan_cached(w, &c)) return DWHIP_OK;
+    const int rc = plan_tune(w, im, 0, nullptr, nullptr);
+    if (rc != DWHIP_OK) {
+        (void)hipGetLastError();  // a failed trial allocation leaves its error behind
+        std::lock_guard<std::mutex> lock(g_cache.mu);
+        load_locked();
+        g_cache.plans[Key{w[0], w[1], w[2]}] = DwhipPlanChoice();
+    }
+    return DWHIP_OK;
+}
+
+extern "C" int dwhip_plan_tune(const int64_t* work, int retune, double* tuned_ms, double* rule_ms)
+{
+    return plan_tune(work, nullptr, retune, tuned_ms, rule_ms);
 }
 
 extern "C" int dwhip_plan_cache_path(const char* path)

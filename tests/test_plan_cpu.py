@@ -57,8 +57,10 @@ def test_trial_image_lies_outside_the_job(probe):
     body = """
         int64_t w[3] = {v[0], v[1], v[2]};
         size_t job = 0, image = 0;
-        dwhip_plan_trial_block(w, &job, &image);
-        const int64_t m[3] = {w[0] / 2, w[1] > 1 ? w[1] / 2 : 1, w[2] > 1 ? w[2] / 2 : 1};
+        const int64_t whole[3] = {v[0], v[1], v[2]};
+        dwhip_plan_trial_block(w, v[3] ? whole : nullptr, &job, &image);
+        int64_t m[3] = {w[0] / 2, w[1] > 1 ? w[1] / 2 : 1, w[2] > 1 ? w[2] / 2 : 1};
+        if (v[3]) m[0] = w[0], m[1] = w[1], m[2] = w[2];
         size_t most = 0;
         for (int x = 0; x <= 1; ++x) {
             DwhipPlanChoice c;
@@ -74,7 +76,8 @@ def test_trial_image_lies_outside_the_job(probe):
         }
         printf("%zu %zu %zu %lld\\n", job, image, most, (long long)(m[0] * m[1] * m[2] * 4));
     """
-    for job, image, most, need in probe(body, FAST):
+    # half the transform, or the job's image (here as large as the transform)
+    for job, image, most, need in probe(body, [w + (whole,) for w in FAST for whole in (0, 1)]):
         assert job % 256 == 0 and most <= job
         assert image >= need
 
