@@ -161,7 +161,7 @@ def preplan(shapes):
             try:
                 dw.plan_tune(w)
             except dw.DwhipError:
-                pass  # sizes the fused passes cannot run keep the any-size path's one plan
+                pass  # sizes the fused passes cannot transform have no plan to measure here
     return time.time() - t
 
 
@@ -356,7 +356,7 @@ def run_c5(fields=1, chunk=4):
 
 def run_anysize():
     """c2 with --bq 1: deconwolf's exact work size (1115 = 5 * 223 along x
-    and y, Bluestein there), timed at 3 and 13 iterations (best of two
+    and y: an extended job, 1296x1296x100), timed at 3 and 13 iterations (best of two
     each); the difference gives the time per iteration."""
     import torch
     import deconwolf_amd as dw
@@ -421,7 +421,7 @@ def main():
                          "that scales rocprofv3 FETCH_SIZE/WRITE_SIZE readings) and exit")
     ap.add_argument("--anysize", action="store_true",
                     help="only time the c2 job at border quality 1 (deconwolf's exact work size 1115x1115x100, "
-                         "the any-size path) at 3 and 13 iterations, print one JSON line and exit")
+                         "an extended job) at 3 and 13 iterations, print one JSON line and exit")
     a = ap.parse_args()
     ENGINE_GROUPS = a.engine_groups
     SERVE_AGING_MS = a.aging_ms
